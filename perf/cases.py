@@ -353,9 +353,11 @@ def run(state):
         return state["call"](state["x"])
     with torch.no_grad():
         snn.functional.reset_net(state["model"])
-        y = state["model"](state["x"]).contiguous()
+        # a plain fp32 tensor: what the next operation outside the fused model
+        # reads (the fused output fills its fp32 form on first use)
+        y = state["model"](state["x"]).detach()
         if case["kind"] == "conv":
-            return y, state["model"][0].state.tensor
+            return y, state["model"][0].state.tensor.detach()
         return y
 
 
