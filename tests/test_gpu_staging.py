@@ -1,0 +1,73 @@
+"""Staging passes between fp32 boundary tensors and the fp16 copies, at the
+edges of their tiles: pixel counts off 64 and off 4, channels off 32 and 64,
+single pixels and channels, values that fp16 cannot hold."""
+import pytest
+import torch
+
+from catfuse_amd import runtime
+
+pytestmark = pytest.mark.gpu
+
+
+def _spikes(shape, cuda, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    n = 1
+    for d in shape:
+        n *= d
+    # (one float into its buffer: contiguous, not 16-byte aligned)
+    x = torch.empty(n + 1, device=cuda)[1:].view(shape)
+    return x.copy_(torch.randint(-3, 4, shape, generator=g))
+
+
+def _status(cuda):
+    return torch.zeros(1, dtype=torch.int32, device=cuda)
+
+
+@pytest.mark.parametrize("shape", [(1, 1, 1, 1), (3, 31, 1, 3), (2, 33, 5, 13), (2, 64, 8, 8),
+                                   (3, 65, 7, 9), (2, 96, 9, 29), (1, 130, 3, 43),
+                                   (5, 200, 45, 61)])
+@pytest.mark.parametrize("act", [False, True])
+def test_pack_input_edges(cuda, shape, act):
+    x = _spikes(shape, cuda)
+    x[x.abs() == 3] *= 0.25                       # quarters: exact in fp16
+    NB, C, H, W = shape
+    gs = max(8, -(-C // 32)) if act else 0
+    nnz = runtime.count_block(x.device)
+    st = _status(cuda)
+    xp, a = runtime.pack_input(x, group_size=gs, nnz=nnz, status=st)
+    want = torch.zeros((NB, H, W, runtime.pad32(C)), device=x.device, dtype=torch.float16)
+    want[..., :C] = x.permute(0, 2, 3, 1).half()
+    assert torch.equal(xp.view(want.shape), want)
+    assert int(nnz[1]) == int((x != 0).sum())
+    if act:
+        bits = torch.zeros((NB, H, W), dtype=torch.int64, device=x.device)
+        for g in range(-(-C // gs)):
+            bits |= (x[:, g * gs:(g + 1) * gs] != 0).any(1).long() << g
+        assert torch.equal(a.view(NB, H, W).long() & 0xffffffff, bits)
+    assert int(st) == 0
+
+
+@pytest.mark.parametrize("rows,C", [(1, 1), (7, 31), (513, 64), (130, 100), (1030, 384)])
+def test_pack_tokens_and_back(cuda, rows, C):
+    x = _spikes((1, 1, rows, C), cuda, 1)
+    cp = runtime.pad32(C)
+    nnz = runtime.count_block(x.device)
+    copy = runtime.pack_tokens(x, cp, nnz=nnz)
+    want = torch.zeros((rows, cp), device=x.device, dtype=torch.float16)
+    want[:, :C] = x.view(rows, C).half()
+    assert torch.equal(copy.view(rows, cp), want)
+    assert int(nnz[1]) == int((x != 0).sum())
+    assert torch.equal(runtime.lazy_tokens((1, 1, rows, C), copy, x.device).clone(), x)
+
+
+@pytest.mark.parametrize("where", [0, 63, 64, 2744 * 70 - 1])
+@pytest.mark.parametrize("bad", [0.1, float("inf"), float("nan"), 1e30])
+def test_pack_flags_what_fp16_cannot_hold(cuda, where, bad):
+    for shape, pack in (((1, 70, 56, 49), runtime.pack_input),
+                        ((1, 1, 2744, 70), lambda x, status: runtime.pack_tokens(x, 96, status=status))):
+        x = torch.zeros(shape, device=cuda)
+        x.view(-1)[where] = bad
+        st = _status(cuda)
+        pack(x, status=st)
+        # an infinity is an fp16 value; what rounds or is no number is not
+        assert int(st) == (0 if bad == float("inf") else runtime.STATUS_INEXACT_FP16)
