@@ -457,6 +457,16 @@ CF_API int cf_conv_halo(const void* x, const void* w_packed, const float* alpha,
                         int epilogue, double tau, double v_th, double v_reset, int hard_reset,
                         int decay_input, void* stream);
 
+// conv_ring.hip
+bool cf_conv_ring(int* rc, const void* x, const void* w_packed, const float* alpha,
+                  const float* beta, const float* v_in, float* v_out, void* out_nhwc,
+                  int64_t cp_out, const void* identity_nhwc, int64_t cp_id,
+                  const unsigned long long* nnz, unsigned long long* nz_out, const void* x_desc,
+                  const void* id_desc, void* out_desc, int bias_info,
+                  const unsigned long long* id_nnz, int64_t T, int64_t B, int64_t Cp,
+                  int64_t Cout, int64_t Coutp, int64_t H, int64_t W, int64_t k, bool pool,
+                  const LifParams& lif, hipStream_t st);
+
 CF_API int cf_conv_mfma(const void* x, const void* w_packed, const float* alpha,
                         const float* beta, const float* v_in, float* v_out, float* out,
                         void* out_nhwc, int64_t cp_out,
@@ -500,6 +510,20 @@ CF_API int cf_conv_mfma(const void* x, const void* w_packed, const float* alpha,
                        (!rect || (tile_h == 8 && (tile_w == 8 ||
                                                   (tile_w == 16 && stride == 1 && KH == 3))));
   if (epilogue == EPI_POOL && !halo_ok) return (int)hipErrorInvalidValue;
+  // Stride-1 1x1 and 3x3 launches without tile masks that write only the
+  // fp16 copy: the flat-tile kernel where it is the faster one (the same
+  // accumulation order, so the same bits).
+  if (!rect && epilogue != EPI_Z && out_nhwc && !out && !identity && stride == 1 &&
+      x_img_tstride == B &&
+      ((KH == 1 && KW == 1 && pad == 0) || (KH == 3 && KW == 3 && pad == 1))) {
+    int rc = 0;
+    if (cf_conv_ring(&rc, x, w_packed, alpha, beta, v_in, v_out, out_nhwc, cp_out, identity_nhwc,
+                     cp_id, nnz, nz_out, x_desc, id_desc, out_desc, bias_info, id_nnz, T, B, Cp,
+                     Cout, Coutp, H, W, KH, epilogue == EPI_POOL,
+                     cf_make_lif_params(tau, v_th, v_reset, hard_reset, decay_input),
+                     (hipStream_t)stream))
+      return rc;
+  }
   if (halo_ok) {
     const int64_t th = 8, tw = rect ? tile_w : 8;
     return cf_conv_halo(x, w_packed, alpha, beta, v_in, v_out, out, out_nhwc, cp_out, identity,

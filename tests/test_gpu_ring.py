@@ -1,0 +1,114 @@
+"""Flat-tile conv kernel (conv_ring.hip) at the edges of its tiles: single
+pixels, maps that leave tiles partly filled or span several images, one chunk
+and odd chunk counts, one to nine time steps, the widest map of each staged
+size, the pooled epilogue; against the CPU oracle, and against the 8x8-tile
+kernel bit for bit (both accumulate in the same order)."""
+import numpy as np
+import pytest
+import torch
+
+import oracle
+from catfuse_amd import runtime
+from catfuse_amd.runtime import EPI_LIF, EPI_POOL, ConvLIFRunner
+from parity import lif_parity
+
+pytestmark = pytest.mark.gpu
+
+# T, B, Cin, Cout, H, W, k: all small enough for one round of workgroups
+SHAPES = [
+    (4, 1, 64, 64, 7, 7, 3), (3, 2, 32, 32, 5, 9, 3), (6, 3, 96, 64, 13, 11, 3),
+    (4, 1, 40, 64, 14, 14, 3), (8, 1, 33, 64, 16, 15, 3), (4, 1, 64, 64, 30, 30, 3),
+    (1, 2, 64, 32, 1, 1, 3), (4, 17, 64, 64, 2, 2, 3), (9, 33, 33, 160, 3, 5, 3),
+    (4, 1, 64, 64, 8, 8, 1), (4, 3, 96, 160, 14, 14, 1), (5, 1, 512, 64, 1, 1, 1),
+    (2, 65, 300, 96, 1, 1, 1), (8, 4, 64, 64, 5, 7, 1), (1, 1, 32, 64, 3, 3, 1),
+    (4, 30, 64, 704, 7, 7, 1),           # 64-channel tiles
+]
+POOLED = [(4, 1, 64, 64, 16, 16), (4, 3, 96, 64, 8, 8), (6, 5, 64, 64, 4, 4),
+          (4, 33, 64, 96, 2, 2), (3, 2, 32, 32, 6, 4), (1, 4, 512, 512, 2, 2)]
+
+
+def _layer(cuda, Ci, Co, k, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    w = torch.randn(Co, Ci, k, k, generator=g) * (2.0 / (Co * k * k)) ** 0.5
+    sc = torch.rand(Co, generator=g) * 0.4 + 0.8
+    sh = torch.randn(Co, generator=g) * 0.1
+    r = ConvLIFRunner(w.to(cuda), sc.to(cuda), sh.to(cuda), None, 1, k // 2, 2.0, 0.3, 0.0, True)
+    return r, w, sc, sh
+
+
+def _lazy(x, cuda):
+    T, B, C, H, W = x.shape
+    xp = runtime.pack_input(x.to(cuda).reshape(T * B, C, H, W))[0]
+    return runtime.lazy_output((T, B, C, H, W), xp, torch.device(cuda))
+
+
+def _tiled(r, x, v0, pool, ident):
+    """The same launch through cf_conv_halo, which the dispatch of
+    cf_conv_mfma passes over."""
+    T, B, Ci, H, W = x.shape
+    dev = x.device
+    xp = x._cf_nhwc[0]
+    Hs, Ws = (H // 2, W // 2) if pool else (H, W)
+    cp = runtime.pad32(r.Cout)
+    out = torch.empty((T * B, Hs, Ws, cp), dtype=torch.float16, device=dev)
+    v = torch.empty((B, r.Cout, Hs, Ws), device=dev)
+    p = runtime.ptr
+    lib = runtime._hip.lib()
+    rc = lib.cf_conv_halo(
+        p(xp), p(r.w_packed), p(r.alpha), p(r.beta), p(v0), p(v), None, p(out), cp, None,
+        p(ident), cp, 1, None, None, None, None, None, None, None, 0, None, x.numel(), 2.0, T, B,
+        r.Cp, r.Cout, r.Coutp, H, W, H, W, r.KH, 1, r.KH // 2, 8, 8, 0,
+        EPI_POOL if pool else EPI_LIF, *r.lif, runtime._hip.stream(dev))
+    assert rc == 0
+    return runtime.lazy_output((T, B, r.Cout, Hs, Ws), out, dev).clone(), v
+
+
+@pytest.mark.parametrize("shape", SHAPES)
+@pytest.mark.parametrize("ident,vin", [(False, False), (True, True)])
+def test_flat_tiles(cuda, shape, ident, vin):
+    T, B, Ci, Co, H, W, k = shape
+    r, w, sc, sh = _layer(cuda, Ci, Co, k)
+    g = torch.Generator().manual_seed(1)
+    x = (torch.rand(T, B, Ci, H, W, generator=g) < 0.3).float()
+    i0 = torch.randint(0, 3, (T, B, Co, H, W), generator=g).float() if ident else None
+    v0 = torch.rand(B, Co, H, W, generator=g) * 0.25 if vin else None
+    xl = _lazy(x, cuda)
+    idl = _lazy(i0, cuda) if ident else None
+    y, v = r.run_mfma(xl, None if v0 is None else v0.to(cuda), identity=idl)
+    y, v = y.clone(), v.clone()
+    ty, tv = _tiled(r, xl, None if v0 is None else v0.to(cuda), False,
+                    idl._cf_nhwc[0] if ident else None)
+    assert torch.equal(y, ty) and torch.equal(v, tv)
+    z = oracle.conv2d(x.reshape(T * B, Ci, H, W), w, None, 1, k // 2)
+    z = torch.as_tensor(np.asarray(z)).reshape(T, B, Co, H, W)
+    z = (z * sc.view(-1, 1, 1) + sh.view(-1, 1, 1)).float()
+    s_ref, v_ref, h_ref = oracle.lif_multistep(z, None if v0 is None else v0, tau=2.0,
+                                               v_threshold=0.3)
+    lif_parity((y - idl.clone() if ident else y).cpu().numpy(), v.cpu().numpy(), s_ref,
+                        v_ref, h_ref, v_th=0.3)
+
+
+@pytest.mark.parametrize("shape", POOLED)
+@pytest.mark.parametrize("vin", [False, True])
+def test_flat_tiles_pooled(cuda, shape, vin):
+    T, B, Ci, Co, H, W = shape
+    r = _layer(cuda, Ci, Co, 3)[0]
+    g = torch.Generator().manual_seed(2)
+    xl = _lazy((torch.rand(T, B, Ci, H, W, generator=g) < 0.3).float(), cuda)
+    v0 = (torch.rand(B, Co, H // 2, W // 2, generator=g) * 0.25).to(cuda) if vin else None
+    y, v = r.run_mfma(xl, v0, epilogue=EPI_POOL)
+    ty, tv = _tiled(r, xl, v0, True, None)
+    assert torch.equal(y.clone(), ty) and torch.equal(v.clone(), tv)
+    assert 0 < float(y.mean()) < 1
+
+
+@pytest.mark.parametrize("k,pool", [(1, False), (3, False), (3, True)])
+def test_flat_tiles_zero_input(cuda, k, pool):
+    """StaticZero: an all-zero input gives the bias response on every route
+    (elided with its count block known, computed without)."""
+    r = _layer(cuda, 64, 64, k)[0]
+    x = torch.zeros(4, 2, 64, 4, 4, device=cuda)
+    r.run_mfma(x, epilogue=EPI_POOL if pool else EPI_LIF)     # bias response known
+    y, v = r.run_mfma(x, epilogue=EPI_POOL if pool else EPI_LIF)
+    ty, tv = _tiled(r, _lazy(x, cuda), None, pool, None)
+    assert torch.equal(y.clone(), ty) and torch.equal(v.clone(), tv)
