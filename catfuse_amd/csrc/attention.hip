@@ -27,6 +27,7 @@ namespace {
 typedef _Float16 h8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef unsigned int u32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned int u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int DH = 32;          // head dim (one MFMA tile edge)
 constexpr int NMAX = 256;       // tokens per image this kernel stages (LDS)
@@ -54,32 +55,36 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t attn_rsrc(const void* base, ui
                                            0x00020000);
 }
 
-template <int LM>
-__global__ __launch_bounds__(256) void spike_attention_kernel(AttnArgs a) {
-  // K and V of the current step, transposed ([d][n], n padded to a
-  // multiple of 16 with zeros) so each MFMA operand is one 16-byte read.
-  // Rows are NMAX + 8 halves apart (528 bytes, 132 dwords: 4 banks on from
-  // the row above), so the 32 rows an operand read touches spread over all
-  // banks instead of sharing four.
-  constexpr int KLD = NMAX + 8;
-  __shared__ __attribute__((aligned(16))) _Float16 kT[DH][KLD];
-  __shared__ __attribute__((aligned(16))) _Float16 vT[DH][KLD];
-  __shared__ __attribute__((aligned(16))) float kvp[4][DH][DH + 1];  // per-wave partial K^T V
-  __shared__ __attribute__((aligned(16))) _Float16 kvT[DH][DH];      // (K^T V)^T as fp16
-  __shared__ unsigned any_sh[4];
+// Every product and sum here is exact (integers), so the order of the sums is
+// free and four time steps run side by side: waves 2 t and 2 t + 1 take step t
+// of the block.  A step's K and V are staged transposed ([d][token], two
+// tokens a word, so each MFMA operand is one 16-byte read; rows of NM / 2 + 4
+// words spread an operand's 32 rows over all banks).  Each wave sums K^T V
+// itself, and its accumulators are the second product's B operand as they
+// lie: the k slots of Y = Q (K^T V) are assigned to the rows d a lane holds,
+// and Q is read in that order.  The sums then meet in LDS (over the staged
+// tokens), and a thread runs the LIF over the block's steps for 8 channels of a
+// token and stores 16 bytes a step.  Bound by latency: one round of loads, one
+// transpose and two barriers a block of four steps, where one step after
+// another took that per step.  Measured (T = 4, 196 tokens, 12 heads): one
+// image 27 -> 14.5 us, 32 images (384 workgroups, one a CU) 39 -> 33.5.
+template <int NM, int LM>
+__global__ __launch_bounds__(512) void spike_attention_kernel(AttnArgs a) {
+  constexpr int TB = 4, KW = NM / 2 + 4, ZLD = DH + 4;
+  constexpr int KV_BYTES = 2 * TB * DH * KW * 4, Z_BYTES = TB * NM * ZLD * 4;
+  constexpr int SU = NM / 64;               // staged units of a thread (2 tokens x 8 channels)
+  constexpr int MAXT = NM / 64;             // 32-token tiles of Y per wave at most
+  constexpr int LU = (NM + 127) / 128;      // LIF units of a thread (a token x 8 channels)
+  __shared__ __attribute__((aligned(16))) char smem[KV_BYTES > Z_BYTES ? KV_BYTES : Z_BYTES];
+  __shared__ unsigned any_sh[8];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hi = lane >> 5, col = lane & 31;
-  const int b = blockIdx.x / a.heads, h = blockIdx.x % a.heads;
+  const int ts = wave >> 1, wh = wave & 1;  // this wave's step of the block, its half of the tiles
   const int N = a.N, C = a.heads * DH;
-  const int NP = (N + 15) & ~15;            // K-dim of K^T V, padded
-  const int nks = NP / 16;                  // its 16-deep MFMA steps
+  const int nks = (N + 15) / 16;            // 16-token MFMA steps of K^T V
   const int ntile = (N + 31) / 32;          // 32-token row tiles of Y
-  // row tiles of this wave: wave, wave + 4
-  constexpr int MAXT = NMAX / 32 / 4;       // row tiles per wave at most
-  float v[MAXT][16];
-  uint32_t anyw = 0u;
   const bool zero_in = a.nnz != nullptr && cf_count_read(a.nnz) == 0ull;   // uniform
   // An all-zero Q/K/V from the initial state drives every neuron with z = 0:
   // when the caller knows that the LIF never fires on it and holds the
@@ -101,134 +106,167 @@ __global__ __launch_bounds__(256) void spike_attention_kernel(AttnArgs a) {
     a.out_desc->vstate = 0u;
     a.out_desc->alias = nullptr;
   }
+  // Neighbouring heads (whose 64-byte rows share cache lines) on one XCD.
+  const int nwork = a.B * a.heads, xcd = (int)blockIdx.x & 7;
+  const int work = xcd * (nwork >> 3) + min(xcd, nwork & 7) + ((int)blockIdx.x >> 3);
+  const int b = work / a.heads, h = work % a.heads;
 
-  // initial membrane potentials
+  // membrane potentials: unit i is token tid / 4 + 128 i, channels 8 (tid % 4) ..
+  const int ln = tid >> 2, lc = (tid & 3) * 8;
+  float v[LU][8];
+  const float v0 = lif_initial_v(a.lif);
 #pragma unroll
-  for (int i = 0; i < MAXT; ++i) {
-    const int tile = wave + 4 * i;
+  for (int i = 0; i < LU; ++i) {
+    const int n = ln + 128 * i;
+    const float* vs = a.v_in + ((size_t)b * N + n) * C + h * DH + lc;
 #pragma unroll
-    for (int r = 0; r < 16; ++r) {
-      const int n = tile * 32 + 8 * (r >> 2) + 4 * hi + (r & 3);
-      float v0 = lif_initial_v(a.lif);
-      if (a.v_in && tile < ntile && n < N) v0 = a.v_in[((size_t)b * N + n) * C + h * DH + col];
-      v[i][r] = v0;
-    }
+    for (int j = 0; j < 8; ++j) v[i][j] = a.v_in != nullptr && n < N ? vs[j] : v0;
   }
+  uint32_t* const kT = reinterpret_cast<uint32_t*>(smem) + ts * 2 * DH * KW;   // [d][pair]
+  uint32_t* const vT = kT + DH * KW;
+  float* const zb = reinterpret_cast<float*>(smem);                            // [t][n][ZLD]
+  uint32_t anyw = 0u;
 
-  for (int t = 0; t < a.T; ++t) {
-    const size_t img = (size_t)t * a.B + b;
-    const _Float16* qb = a.q + img * N * a.pitch + a.qoff + h * DH;
-    const _Float16* kb = a.k + img * N * a.pitch + a.koff + h * DH;
-    const _Float16* vb = a.v + img * N * a.pitch + a.voff + h * DH;
-    // this step's Q rows (A operand: row tile*32 + col, k 16 hi ..), issued
-    // first so their latency overlaps the K^T V phase; rows beyond N read
-    // zeros (out of the buffer's range)
-    const __amdgpu_buffer_rsrc_t rq = attn_rsrc(qb, (uint32_t)(((size_t)(N - 1) * a.pitch + DH) * 2));
-    h8 qr[MAXT][2];
-    h8 kv0 = {}, kv1 = {};
+  for (int tb0 = 0; tb0 < a.T; tb0 += TB) {
+    const int nst = min(TB, a.T - tb0);
+    f32x16 y[MAXT];
+#pragma unroll
+    for (int i = 0; i < MAXT; ++i) y[i] = f32x16{};
     if (!zero_in) {
+      // (steps beyond the last read step 0's rows and are not used)
+      const size_t img = (size_t)(ts < nst ? tb0 + ts : 0) * a.B + b;
+      const uint32_t bytes = (uint32_t)(((size_t)(N - 1) * a.pitch + DH) * 2);
+      const __amdgpu_buffer_rsrc_t rq = attn_rsrc(a.q + img * N * a.pitch + a.qoff + h * DH, bytes);
+      const __amdgpu_buffer_rsrc_t rk = attn_rsrc(a.k + img * N * a.pitch + a.koff + h * DH, bytes);
+      const __amdgpu_buffer_rsrc_t rv = attn_rsrc(a.v + img * N * a.pitch + a.voff + h * DH, bytes);
+      // every load of the block is issued before its first use (rows beyond
+      // N read zeros, out of the buffers' range)
+      auto off = [&](int n, int c) { return n < N ? (uint32_t)((n * a.pitch + c) * 2) : 0x80000000u; };
+      const int g = tid & 127;
+      u32x4 kx[SU][2], vx[SU][2];
+#pragma unroll
+      for (int i = 0; i < SU; ++i) {
+        const int u = g + 128 * i, n = (u >> 2) * 2, c = (u & 3) * 8;
+#pragma unroll
+        for (int e = 0; e < 2; ++e) {
+          kx[i][e] = __builtin_amdgcn_raw_buffer_load_b128(rk, off(n + e, c), 0, 0);
+          vx[i][e] = __builtin_amdgcn_raw_buffer_load_b128(rv, off(n + e, c), 0, 0);
+        }
+      }
+      // Q rows of this wave's tiles: k slots (hi, 0..3) and (hi, 4..7) of MFMA
+      // step s are channels 16 s + 4 hi .. + 3 and 16 s + 8 + 4 hi .. + 3
+      u32x2 qx[MAXT][2][2];
+#pragma unroll
+      for (int i = 0; i < MAXT; ++i)
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+          for (int e = 0; e < 2; ++e)
+            qx[i][s][e] = __builtin_amdgcn_raw_buffer_load_b64(
+                rq, off((wh + 2 * i) * 32 + col, 16 * s + 8 * e + 4 * hi), 0, 0);
+#pragma unroll
+      for (int i = 0; i < SU; ++i) {
+        const int u = g + 128 * i, pr = u >> 2, c = (u & 3) * 8;
+        if (2 * pr < 16 * nks) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            const uint32_t sel = (j & 1) ? 0x07060302u : 0x05040100u;   // high / low halves
+            kT[(c + j) * KW + pr] = __builtin_amdgcn_perm(kx[i][1][j >> 1], kx[i][0][j >> 1], sel);
+            vT[(c + j) * KW + pr] = __builtin_amdgcn_perm(vx[i][1][j >> 1], vx[i][0][j >> 1], sel);
+          }
+        }
+      }
+      __syncthreads();
+      f32x16 kv = {};
+      for (int s = 0; s < nks; ++s) {
+        const h8 av = *reinterpret_cast<const h8*>(&kT[col * KW + 8 * s + 4 * hi]);
+        const h8 bv = *reinterpret_cast<const h8*>(&vT[col * KW + 8 * s + 4 * hi]);
+        kv = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, bv, kv, 0, 0, 0);
+      }
+      h8 kvb[2];   // entries <= N: exact in fp16
+#pragma unroll
+      for (int s = 0; s < 2; ++s)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) kvb[s][j] = (_Float16)kv[8 * s + j];
+#pragma unroll
+      for (int i = 0; i < MAXT; ++i)
+#pragma unroll
+        for (int s = 0; s < 2; ++s) {
+          const u32x4 q4 = {qx[i][s][0][0], qx[i][s][0][1], qx[i][s][1][0], qx[i][s][1][1]};
+          y[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(h8, q4), kvb[s], y[i], 0,
+                                                        0, 0);
+        }
+      __syncthreads();   // kT and vT are read: the sums take their place
+    }
 #pragma unroll
     for (int i = 0; i < MAXT; ++i) {
-      const int n = (wave + 4 * i) * 32 + col;
-      const uint32_t qo = n < N ? (uint32_t)(((size_t)n * a.pitch) * 2) : 0x80000000u;
-      qr[i][0] = __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(rq, qo + 16 * hi, 0, 0));
-      qr[i][1] = __builtin_bit_cast(h8, __builtin_amdgcn_raw_buffer_load_b128(rq, qo + 32 + 16 * hi, 0, 0));
-    }
-    __syncthreads();  // the previous step's reads of kT / vT / kvT are complete
-    // stage K, V transposed: unit u = tid + 256 i = (token u / 4, 8-channel
-    // part u % 4); every load of the thread is issued before the first LDS
-    // write, so the step waits for one load latency, not one per unit
-    constexpr int SU = NMAX * 4 / 256;
-    h8 kx[SU], vx[SU];
+      const int tile = wh + 2 * i;
+      if (tile >= ntile) break;
 #pragma unroll
-    for (int i = 0; i < SU; ++i) {
-      const int u = tid + 256 * i, n = u >> 2, c = (u & 3) * 8;
-      kx[i] = h8{};
-      vx[i] = h8{};
-      if (n < N) {
-        kx[i] = *reinterpret_cast<const h8*>(kb + (size_t)n * a.pitch + c);
-        vx[i] = *reinterpret_cast<const h8*>(vb + (size_t)n * a.pitch + c);
-      }
+      for (int r = 0; r < 16; ++r)
+        zb[(ts * NM + tile * 32 + 8 * (r >> 2) + 4 * hi + (r & 3)) * ZLD + col] = y[i][r];
     }
+    __syncthreads();
 #pragma unroll
-    for (int i = 0; i < SU; ++i) {
-      const int u = tid + 256 * i, n = u >> 2, c = (u & 3) * 8;
-      if (n < NP) {
+    for (int i = 0; i < LU; ++i) {
+      const int n = ln + 128 * i;
+      if (n >= N) break;
+#pragma unroll
+      for (int t = 0; t < TB; ++t) {
+        if (t >= nst) break;
+        const float* zp = &zb[(t * NM + n) * ZLD + lc];
+        h8 sp;
 #pragma unroll
         for (int j = 0; j < 8; ++j) {
-          kT[c + j][n] = kx[i][j];
-          vT[c + j][n] = vx[i][j];
+          const float z = zp[j] * a.scale;
+          float vv = lif_charge_m<LM>(v[i][j], z, a.lif);
+          sp[j] = lif_fire_reset_bit<LM>(vv, a.lif) ? (_Float16)1.0f : (_Float16)0.0f;
+          v[i][j] = vv;
+        }
+        const u32x4 w = __builtin_bit_cast(u32x4, sp);
+        anyw |= w[0] | w[1] | w[2] | w[3];
+        _Float16* o = a.out + (((size_t)(tb0 + t) * a.B + b) * N + n) * a.cp_out + h * DH + lc;
+        if (a.cp_out % 8 == 0 && ((uintptr_t)a.out & 15) == 0) {
+          *reinterpret_cast<u32x4*>(o) = w;
+        } else {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) o[j] = sp[j];
         }
       }
     }
-    __syncthreads();
-    // K^T V: wave w accumulates the K steps w, w + 4, ...
-    {
-      f32x16 acc = {};
-      for (int s = wave; s < nks; s += 4) {
-        const int n0 = s * 16 + 8 * hi;
-        const h8 av = *reinterpret_cast<const h8*>(&kT[col][n0]);   // A[i = col][n]
-        const h8 bv = *reinterpret_cast<const h8*>(&vT[col][n0]);   // B[n][j = col]
-        acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(av, bv, acc, 0, 0, 0);
-      }
-#pragma unroll
-      for (int r = 0; r < 16; ++r) kvp[wave][8 * (r >> 2) + 4 * hi + (r & 3)][col] = acc[r];
-    }
-    __syncthreads();
-    // sum the partials (integers: exact in any order) and keep (K^T V)^T in
-    // fp16 (entries <= N, exact): kvT[j][i] = KV[i][j]
-    for (int e = tid; e < DH * DH; e += 256) {
-      const int i = e >> 5, j = e & 31;
-      const float s = kvp[0][i][j] + kvp[1][i][j] + kvp[2][i][j] + kvp[3][i][j];
-      kvT[j][i] = (_Float16)s;
-    }
-    __syncthreads();
-    // Y = Q KV per 32-token row tile; B operand: KV[i][j = col] for i in the step
-    kv0 = *reinterpret_cast<const h8*>(&kvT[col][8 * hi]);
-    kv1 = *reinterpret_cast<const h8*>(&kvT[col][16 + 8 * hi]);
-    }  // !zero_in
-    _Float16* ob = a.out + img * N * a.cp_out + h * DH;
-#pragma unroll
-    for (int i = 0; i < MAXT; ++i) {
-      const int tile = wave + 4 * i;
-      if (tile >= ntile) break;
-      f32x16 y = {};
-      if (!zero_in) {
-        y = __builtin_amdgcn_mfma_f32_32x32x16_f16(qr[i][0], kv0, y, 0, 0, 0);
-        y = __builtin_amdgcn_mfma_f32_32x32x16_f16(qr[i][1], kv1, y, 0, 0, 0);
-      }
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int nr = tile * 32 + 8 * (r >> 2) + 4 * hi + (r & 3);
-        const float z = y[r] * a.scale;
-        float vv = lif_charge_m<LM>(v[i][r], z, a.lif);
-        const bool f = lif_fire_reset_bit<LM>(vv, a.lif);
-        v[i][r] = vv;
-        if (nr < N) {
-          ob[(size_t)nr * a.cp_out + col] = f ? (_Float16)1.0f : (_Float16)0.0f;
-          anyw |= f ? 1u : 0u;
-        }
-      }
-    }
+    if (tb0 + TB < a.T) __syncthreads();   // the sums are read: the next block stages here
   }
   if (a.v_out) {
 #pragma unroll
-    for (int i = 0; i < MAXT; ++i) {
-      const int tile = wave + 4 * i;
-      if (tile >= ntile) break;
+    for (int i = 0; i < LU; ++i) {
+      const int n = ln + 128 * i;
+      if (n >= N) break;
+      float* vd = a.v_out + ((size_t)b * N + n) * C + h * DH + lc;
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int n = tile * 32 + 8 * (r >> 2) + 4 * hi + (r & 3);
-        if (n < N) a.v_out[((size_t)b * N + n) * C + h * DH + col] = v[i][r];
-      }
+      for (int j = 0; j < 8; ++j) vd[j] = v[i][j];
     }
   }
   if (a.nz_out) {
-    const bool any = cf_wg_any(anyw != 0u, any_sh);
-    if (tid == 0) cf_count_publish(a.nz_out, any ? 1ull : 0ull, blockIdx.x, gridDim.x);
+    const bool any = __any(anyw != 0u ? 1 : 0) != 0;
+    if (lane == 0) any_sh[wave] = any ? 1u : 0u;
+    __syncthreads();
+    if (tid == 0) {
+      unsigned w = 0u;
+#pragma unroll
+      for (int i = 0; i < 8; ++i) w |= any_sh[i];
+      cf_count_publish(a.nz_out, w ? 1ull : 0ull, blockIdx.x, gridDim.x);
+    }
   }
 }
 
+// (Workgroups of fewer tokens need less LDS, so more share a CU.)
+template <int LM>
+void launch_attention(const AttnArgs& a, hipStream_t st) {
+  const dim3 grid((unsigned)(a.B * a.heads)), block(512);
+  if (a.N <= 64) hipLaunchKernelGGL((spike_attention_kernel<64, LM>), grid, block, 0, st, a);
+  else if (a.N <= 128) hipLaunchKernelGGL((spike_attention_kernel<128, LM>), grid, block, 0, st, a);
+  else hipLaunchKernelGGL((spike_attention_kernel<NMAX, LM>), grid, block, 0, st, a);
+}
 
 // ---------------------------------------------------------------------------
 // Two-pass form for any token count and head dims 32 or 64.
@@ -488,15 +526,11 @@ CF_API int cf_spike_attention_lif(const void* q, const void* k, const void* v, i
   a.out_desc = (CfOutDesc*)out_desc; a.zero_info = zero_info; a.B = (int)B; a.N = (int)N; a.heads = (int)heads;
   a.scale = (float)scale;
   a.lif = cf_make_lif_params(tau, v_th, v_reset, hard_reset, decay_input);
-  const dim3 grid((unsigned)(B * heads)), block(256);
   const int lm = cf_lif_mode(a.lif);
   hipStream_t st = (hipStream_t)stream;
-  if (lm == LM_HARD0_DECAY_P2)
-    hipLaunchKernelGGL(spike_attention_kernel<LM_HARD0_DECAY_P2>, grid, block, 0, st, a);
-  else if (lm == LM_HARD_DECAY_P2)
-    hipLaunchKernelGGL(spike_attention_kernel<LM_HARD_DECAY_P2>, grid, block, 0, st, a);
-  else
-    hipLaunchKernelGGL(spike_attention_kernel<LM_GENERIC>, grid, block, 0, st, a);
+  if (lm == LM_HARD0_DECAY_P2) launch_attention<LM_HARD0_DECAY_P2>(a, st);
+  else if (lm == LM_HARD_DECAY_P2) launch_attention<LM_HARD_DECAY_P2>(a, st);
+  else launch_attention<LM_GENERIC>(a, st);
   return (int)hipGetLastError();
 }
 
