@@ -453,6 +453,12 @@ __global__ __launch_bounds__(256) void linear_tokens_kernel(
 // positions ignored, as torch's max_pool2d) of xp[n][ih][iw][c].  The max of
 // spike values is exact in fp16.  One 8-channel chunk of one output pixel
 // per thread; the nonzero count of the output is published (count block).
+// KC, SC, PC: the window, stride and padding of the usual pool (3, 2, 1), whose
+// nine loads are then in flight together (a window position outside the
+// input repeats the centre, which is inside it and changes no maximum); 0: as
+// the arguments say.  32 x 112 x 112 x 96: 32 -> 26 us, 32 x 56 x 56 x 192
+// 20.6 -> 13.6, 4 x 28 x 28 x 384 8.2 -> 4.6.
+template <int KC, int SC, int PC>
 __global__ __launch_bounds__(256) void maxpool_nhwc_kernel(
     const _Float16* __restrict__ xp_own, const CfOutDesc* __restrict__ in_desc,
     _Float16* __restrict__ out, CfOutDesc* __restrict__ out_desc, int64_t NB, int H, int W,
@@ -489,6 +495,27 @@ __global__ __launch_bounds__(256) void maxpool_nhwc_kernel(
     const int oh = (int)(r / (uint32_t)Wo), ow = (int)(r - (uint32_t)oh * (uint32_t)Wo);
     const int64_t n = n32;
     h8 m;
+    if constexpr (KC != 0) {
+      static_assert(PC < KC && SC <= KC, "the window's centre lies inside the input");
+      h8 v[KC * KC];
+#pragma unroll
+      for (int dy = 0; dy < KC; ++dy)
+#pragma unroll
+        for (int dx = 0; dx < KC; ++dx) {
+          int ih = oh * SC - PC + dy, iw = ow * SC - PC + dx;
+          if (ih < 0 || ih >= H) ih = oh * SC - PC + KC / 2;
+          if (iw < 0 || iw >= W) iw = ow * SC - PC + KC / 2;
+          v[dy * KC + dx] =
+              xp != nullptr
+                  ? *reinterpret_cast<const h8*>(xp + ((n * H + ih) * W + iw) * cp + c8 * 8)
+                  : h8{};
+        }
+      m = v[0];
+#pragma unroll
+      for (int q = 1; q < KC * KC; ++q)
+#pragma unroll
+        for (int j = 0; j < 8; ++j) m[j] = v[q][j] > m[j] ? v[q][j] : m[j];
+    } else {
     bool first = true;
     for (int dy = 0; dy < k; ++dy) {
       const int ih = oh * s - p + dy;
@@ -507,6 +534,7 @@ __global__ __launch_bounds__(256) void maxpool_nhwc_kernel(
           for (int j = 0; j < 8; ++j) m[j] = v[j] > m[j] ? v[j] : m[j];
         }
       }
+    }
     }
     const uint4 w = __builtin_bit_cast(uint4, m);
     anyw |= (w.x | w.y | w.z | w.w) & 0x7fff7fffu;
@@ -738,10 +766,18 @@ CF_API int cf_maxpool_nhwc(const void* xp, const void* in_desc, void* out, void*
   if (units >= ((int64_t)1 << 31)) return (int)hipErrorInvalidValue;   // 32-bit unit indices
   // about one unit a thread (more loads in flight than a grid-stride loop)
   const unsigned grid = (unsigned)((units + 255) / 256 < 65536 ? (units + 255) / 256 : 65536);
-  hipLaunchKernelGGL(maxpool_nhwc_kernel, dim3(grid), dim3(256), 0, (hipStream_t)stream,
-                     (const _Float16*)xp, (const CfOutDesc*)in_desc, (_Float16*)out,
-                     (CfOutDesc*)out_desc, NB, (int)H, (int)W, (int)Ho, (int)Wo,
-                     (int)cp, (int)kernel_size, (int)stride, (int)padding, nz_out);
+  // (floor mode: the centre of a (3, 2, 1) window, row 2 oh and column 2 ow,
+  // is inside the input)
+  if (kernel_size == 3 && stride == 2 && padding == 1)
+    hipLaunchKernelGGL((maxpool_nhwc_kernel<3, 2, 1>), dim3(grid), dim3(256), 0,
+                       (hipStream_t)stream, (const _Float16*)xp, (const CfOutDesc*)in_desc,
+                       (_Float16*)out, (CfOutDesc*)out_desc, NB, (int)H, (int)W, (int)Ho, (int)Wo,
+                       (int)cp, 3, 2, 1, nz_out);
+  else
+    hipLaunchKernelGGL((maxpool_nhwc_kernel<0, 0, 0>), dim3(grid), dim3(256), 0,
+                       (hipStream_t)stream, (const _Float16*)xp, (const CfOutDesc*)in_desc,
+                       (_Float16*)out, (CfOutDesc*)out_desc, NB, (int)H, (int)W, (int)Ho, (int)Wo,
+                       (int)cp, (int)kernel_size, (int)stride, (int)padding, nz_out);
   return (int)hipGetLastError();
 }
 
