@@ -129,12 +129,22 @@ __global__ __launch_bounds__(256) void conv_direct_kernel(DirectArgs a) {
 // read transposed ([Cin*9][Cout]) so each filter tap is one wave-uniform
 // read of COB consecutive floats.  z is the same fp32 fused multiply-add
 // chain as conv_direct_kernel's, so the spikes are bit-identical to
-// conv_direct_kernel followed by the pool.  Per step each thread stores the
-// COB spike bits of its conv output as one 64-bit word; a pooled output is
-// the OR of the nine words of its window (the max of {0, 1} values; the
-// pool's -inf padding never wins because every window holds a conv output).
+// conv_direct_kernel followed by the pool.  Per block of four steps each
+// thread stores its conv output's spikes as four bits a channel, eight channels
+// a word; a pooled output is the OR of the nine words of its window (the max of
+// {0, 1} values; the pool's -inf padding never wins because every window
+// holds a conv output), one pass over the windows for all four steps.
 // v_out keeps the final membrane of the conv outputs the tile owns (local
 // rows and columns >= 1).
+//
+// Bound by vector instructions: 27 multiply-adds and four LIF steps for every
+// channel of 1.14 conv outputs a pixel.  FAST (the stage as a network runs it: the
+// same image at T = 4 steps from the initial state, a hard reset) takes the
+// four potentials as reset-free charges u1 .. u4: a reset returns v to its
+// initial value bit for bit, so with k the first step where u_k >= v_th the
+// neuron fires at k, 2 k, ... and ends at u_(4 mod k).  8 images of 224 x 224,
+// 48 channels: 72 us (a window pass and a barrier every step, stepped LIF) ->
+// 61.5, with the filter read through scalar registers and the staged tile's loads together.
 constexpr int DP_PH = 7, DP_PW = 8;                  // pooled tile
 constexpr int DP_RH = 2 * DP_PH + 1, DP_RW = 2 * DP_PW + 1;   // 15 x 17 conv outputs
 constexpr int DP_NPIX = DP_RH * DP_RW;               // 255
@@ -155,12 +165,13 @@ struct DirectPoolArgs {
   LifParams lif;
 };
 
-template <int COB, int LM>
+template <int COB, int LM, bool FAST>
 __global__ __launch_bounds__(256) void conv_direct_pool_kernel(DirectPoolArgs a) {
-  static_assert(COB % 8 == 0 && COB <= 64, "COB spike bits per 64-bit word");
+  static_assert(COB % 8 == 0 && COB <= 64, "8 channels a word");
+  static_assert(!FAST || LM == LM_HARD0_DECAY_P2, "reset-free charges: a hard reset to +0");
+  constexpr int NWD = COB / 8;
   __shared__ float xs[DP_MAXCIN][DP_XH][DP_XW];
-  __shared__ __attribute__((aligned(16))) float wsm[DP_MAXCIN * 9][COB];   // [tap][channel]
-  __shared__ unsigned long long spk[2][256];
+  __shared__ uint32_t spk[2][NWD][256];
   __shared__ unsigned any_sh[4];
   const int tid = threadIdx.x;
   const int b = blockIdx.y, co0 = blockIdx.z * COB;
@@ -186,21 +197,28 @@ __global__ __launch_bounds__(256) void conv_direct_pool_kernel(DirectPoolArgs a)
     for (int j = 0; j < COB; ++j) v[j] = lif_initial_v(a.lif);
   }
   uint32_t anyw = 0u;
-  // this workgroup's filter slice; every lane reads the same weights, so
-  // the conv reads them as LDS broadcasts (16 bytes, four channels, a read)
-  for (int u = tid; u < a.Cin * 9 * COB; u += 256)
-    wsm[u / COB][u % COB] = a.wt[(size_t)(u / COB) * a.Cout + co0 + u % COB];
-  for (int t = 0; t < a.T; ++t) {
-    if (t == 0 || !dedupe) {
+  // this workgroup's filter slice, read through scalar registers (every lane
+  // multiplies by the same weights)
+  typedef const __attribute__((address_space(4))) float cfloat;
+  cfloat* const wc = (cfloat*)(uintptr_t)(a.wt + co0);
+  auto conv_step = [&](int t) {
       const int img = t * a.x_img_tstride + b;
       if (t > 0) __syncthreads();   // the previous step's reads of xs are complete
       const float* xb = a.x + (size_t)img * a.Cin * a.H * a.W;
-      for (int u = tid; u < a.Cin * DP_XH * DP_XW; u += 256) {
-        const int ci = u / (DP_XH * DP_XW), rr = (u / DP_XW) % DP_XH, c = u % DP_XW;
+      // (every load of the tile in flight before the first is stored)
+      constexpr int SU = (DP_MAXCIN * DP_XH * DP_XW + 255) / 256;
+      float st[SU];
+#pragma unroll
+      for (int i = 0; i < SU; ++i) {
+        const int u = tid + 256 * i;
+        const int ci = u / (DP_XH * DP_XW), rr = u / DP_XW - ci * DP_XH, c = u % DP_XW;
         const int ih = cr0 - a.pad + rr, iw = cc0 - a.pad + c;
-        xs[ci][rr][c] = (ih >= 0 && ih < a.H && iw >= 0 && iw < a.W)
-                            ? xb[((size_t)ci * a.H + ih) * a.W + iw] : 0.0f;
+        const bool in = ci < a.Cin && ih >= 0 && ih < a.H && iw >= 0 && iw < a.W;
+        st[i] = in ? xb[((size_t)ci * a.H + ih) * a.W + iw] : 0.0f;
       }
+#pragma unroll
+      for (int i = 0; i < SU; ++i)
+        if (tid + 256 * i < a.Cin * DP_XH * DP_XW) (&xs[0][0][0])[tid + 256 * i] = st[i];
       __syncthreads();
       float acc[COB];
 #pragma unroll
@@ -211,30 +229,65 @@ __global__ __launch_bounds__(256) void conv_direct_pool_kernel(DirectPoolArgs a)
 #pragma unroll
           for (int kw = 0; kw < 3; ++kw) {
             const float xv = xs[ci][lr + kh][lc + kw];
-            const float4* wk = reinterpret_cast<const float4*>(wsm[(ci * 3 + kh) * 3 + kw]);
+            cfloat* const wk = wc + ((ci * 3 + kh) * 3 + kw) * a.Cout;
 #pragma unroll
-            for (int j = 0; j < COB; j += 4) {
-              const float4 w4 = wk[j / 4];
-              acc[j] = fmaf(xv, w4.x, acc[j]);
-              acc[j + 1] = fmaf(xv, w4.y, acc[j + 1]);
-              acc[j + 2] = fmaf(xv, w4.z, acc[j + 2]);
-              acc[j + 3] = fmaf(xv, w4.w, acc[j + 3]);
-            }
+            for (int j = 0; j < COB; ++j) acc[j] = fmaf(xv, wk[j], acc[j]);
           }
         }
       }
 #pragma unroll
       for (int j = 0; j < COB; ++j) z[j] = fmaf(acc[j], a.alpha[co0 + j], a.beta[co0 + j]);
-    }
-    unsigned long long m = 0ull;
+  };
+  for (int tb0 = 0; tb0 < a.T; tb0 += 4) {
+    const int nst = FAST ? 4 : min(4, a.T - tb0);
+    uint32_t m[NWD];   // four bits (steps) of eight channels a word
 #pragma unroll
-    for (int j = 0; j < COB; ++j) {
-      float vv = lif_charge_m<LM>(v[j], z[j], a.lif);
-      const bool f = lif_fire_reset_bit<LM>(vv, a.lif);
-      v[j] = vv;
-      m |= (f ? 1ull : 0ull) << j;
+    for (int i = 0; i < NWD; ++i) m[i] = 0u;
+    if constexpr (FAST) {
+      conv_step(0);
+#pragma unroll
+      for (int j = 0; j < COB; ++j) {
+        const float u1 = lif_charge_m<LM>(v[j], z[j], a.lif);
+        const float u2 = lif_charge_m<LM>(u1, z[j], a.lif);
+        const float u3 = lif_charge_m<LM>(u2, z[j], a.lif);
+        const float u4 = lif_charge_m<LM>(u3, z[j], a.lif);
+        // The reset's value is +0; an infinite potential (only an infinite z
+        // gives one, at once: the host admits |1 / tau| <= 1) resets to
+        // 0 * inf = NaN and never fires again.  One compare and its two selects
+        // at a time (left to itself the compiler combines the compares of many
+        // channels, whose masks then spill out of the scalar registers).
+        const float r0 = __builtin_fmaf(0.0f, u1, 0.0f);
+        uint32_t q1 = 0xfu, q = 0u;
+        float vf = u4;
+        auto pin = [&]() { asm volatile("" : "+v"(vf), "+v"(q), "+v"(q1)); };
+        q1 = r0 == 0.0f ? q1 : 0x1u;
+        pin();
+        { const bool f = u4 >= a.lif.v_th; vf = f ? 0.0f : vf; q = f ? 0x8u : q; }
+        pin();
+        { const bool f = u3 >= a.lif.v_th; vf = f ? u1 : vf; q = f ? 0x4u : q; }
+        pin();
+        { const bool f = u2 >= a.lif.v_th; vf = f ? 0.0f : vf; q = f ? 0xau : q; }
+        pin();
+        { const bool f = u1 >= a.lif.v_th; vf = f ? r0 : vf; q = f ? q1 : q; }
+        pin();
+        m[j / 8] |= q << (4 * (j % 8));
+        v[j] = vf;
+      }
+    } else {
+      for (int t = 0; t < nst; ++t) {
+        if (tb0 + t == 0 || !dedupe) conv_step(tb0 + t);
+#pragma unroll
+        for (int j = 0; j < COB; ++j) {
+          float vv = lif_charge_m<LM>(v[j], z[j], a.lif);
+          const bool f = lif_fire_reset_bit<LM>(vv, a.lif);
+          v[j] = vv;
+          m[j / 8] |= (f ? 1u : 0u) << (4 * (j % 8) + t);
+        }
+      }
     }
-    spk[t & 1][tid] = valid ? m : 0ull;
+    const int sb = (tb0 >> 2) & 1;
+#pragma unroll
+    for (int i = 0; i < NWD; ++i) spk[sb][i][tid] = valid ? m[i] : 0u;
     __syncthreads();
     // pooled outputs: unit = (pooled pixel of the tile, 16-byte chunk)
     for (int u = tid; u < DP_PH * DP_PW * nch; u += 256) {
@@ -243,22 +296,28 @@ __global__ __launch_bounds__(256) void conv_direct_pool_kernel(DirectPoolArgs a)
       const int gy = ph0 + py, gx = pw0 + px;
       if (gy >= a.Hp || gx >= a.Wp) continue;
       uint32_t bits = 0u;
-      if (ch * 8 < COB) {
-        unsigned long long w = 0ull;
+      if (ch < NWD) {
 #pragma unroll
         for (int dy = 0; dy < 3; ++dy)
 #pragma unroll
-          for (int dx = 0; dx < 3; ++dx) w |= spk[t & 1][(2 * py + dy) * DP_RW + 2 * px + dx];
-        bits = (uint32_t)(w >> (ch * 8)) & 0xffu;
+          for (int dx = 0; dx < 3; ++dx) bits |= spk[sb][ch][(2 * py + dy) * DP_RW + 2 * px + dx];
       }
       anyw |= bits;
-      uint4 o;
-      o.x = ((bits & 1u) ? 0x3c00u : 0u) | ((bits & 2u) ? 0x3c000000u : 0u);
-      o.y = ((bits & 4u) ? 0x3c00u : 0u) | ((bits & 8u) ? 0x3c000000u : 0u);
-      o.z = ((bits & 16u) ? 0x3c00u : 0u) | ((bits & 32u) ? 0x3c000000u : 0u);
-      o.w = ((bits & 64u) ? 0x3c00u : 0u) | ((bits & 128u) ? 0x3c000000u : 0u);
-      *reinterpret_cast<uint4*>(a.out_nhwc + (((size_t)t * a.B + b) * a.Hp + gy) * a.Wp * a.cp_out +
-                                (size_t)gx * a.cp_out + co0 + ch * 8) = o;
+      _Float16* o = a.out_nhwc + (((size_t)tb0 * a.B + b) * a.Hp + gy) * a.Wp * a.cp_out +
+                    (size_t)gx * a.cp_out + co0 + ch * 8;
+      const size_t tstr = (size_t)a.B * a.Hp * a.Wp * a.cp_out;
+#pragma unroll
+      for (int t = 0; t < 4; ++t) {
+        if (t >= nst) break;
+        // channel j's bit of step t is bit 4 j + t; 0x3c00 is fp16 1.0
+        auto pair = [&](int j) -> uint32_t {
+          const uint32_t lo = (uint32_t)((int32_t)(bits << (31 - 4 * j - t)) >> 31);
+          const uint32_t hi = (uint32_t)((int32_t)(bits << (27 - 4 * j - t)) >> 31);
+          return (lo & 0x3c00u) | (hi & 0x3c000000u);
+        };
+        const uint4 q = make_uint4(pair(0), pair(2), pair(4), pair(6));
+        *reinterpret_cast<uint4*>(o + t * tstr) = q;
+      }
     }
   }
   if (a.v_out && valid && lr >= 1 && lc >= 1) {
@@ -457,14 +516,17 @@ __global__ __launch_bounds__(256) void conv_direct_avgpool_kernel(DirectAvgArgs 
   }
 }
 
-template <int LM>
-hipError_t launch_direct_pool(const DirectPoolArgs& a, int cob, dim3 grid, hipStream_t st) {
-  switch (cob) {
-    case 64: hipLaunchKernelGGL((conv_direct_pool_kernel<64, LM>), grid, dim3(256), 0, st, a); break;
-    case 48: hipLaunchKernelGGL((conv_direct_pool_kernel<48, LM>), grid, dim3(256), 0, st, a); break;
-    case 32: hipLaunchKernelGGL((conv_direct_pool_kernel<32, LM>), grid, dim3(256), 0, st, a); break;
-    default: hipLaunchKernelGGL((conv_direct_pool_kernel<16, LM>), grid, dim3(256), 0, st, a); break;
-  }
+hipError_t launch_direct_pool(const DirectPoolArgs& a, dim3 grid, hipStream_t st) {
+  const int lm = cf_lif_mode(a.lif);
+  const bool fast = lm == LM_HARD0_DECAY_P2 && a.T == 4 && a.x_img_tstride == 0 && !a.v_in &&
+                    a.lif.inv_tau > 0.0f && a.lif.inv_tau <= 1.0f;
+#define CF_DIRECT_POOL(LMV, F) \
+  hipLaunchKernelGGL((conv_direct_pool_kernel<16, LMV, F>), grid, dim3(256), 0, st, a)
+  if (fast) CF_DIRECT_POOL(LM_HARD0_DECAY_P2, true);
+  else if (lm == LM_HARD0_DECAY_P2) CF_DIRECT_POOL(LM_HARD0_DECAY_P2, false);
+  else if (lm == LM_HARD_DECAY_P2) CF_DIRECT_POOL(LM_HARD_DECAY_P2, false);
+  else CF_DIRECT_POOL(LM_GENERIC, false);
+#undef CF_DIRECT_POOL
   return hipGetLastError();
 }
 
@@ -541,11 +603,7 @@ CF_API int cf_conv_direct_lif_maxpool(const float* x, const float* wt, const flo
   a.tiles_w = (int)tiles_w; a.x_img_tstride = (int)x_img_tstride;
   a.lif = cf_make_lif_params(tau, v_th, v_reset, hard_reset, decay_input);
   const dim3 grid((unsigned)(tiles_h * tiles_w), (unsigned)B, (unsigned)(Cout / cob));
-  const int lm = cf_lif_mode(a.lif);
-  hipStream_t st = (hipStream_t)stream;
-  if (lm == LM_HARD0_DECAY_P2) return (int)launch_direct_pool<LM_HARD0_DECAY_P2>(a, cob, grid, st);
-  if (lm == LM_HARD_DECAY_P2) return (int)launch_direct_pool<LM_HARD_DECAY_P2>(a, cob, grid, st);
-  return (int)launch_direct_pool<LM_GENERIC>(a, cob, grid, st);
+  return (int)launch_direct_pool(a, grid, (hipStream_t)stream);
 }
 
 // Conv(3 x 3, stride 1, Cin <= 4) -> BN -> AvgPool2d(2, 2) -> LIF of an
