@@ -125,6 +125,12 @@ __device__ __forceinline__ float lif_initial_v(const LifParams& p) {
   return p.hard ? p.v_reset : 0.0f;
 }
 
+// Whether a neuron in its initial state stays there, silent, under z = 0: the
+// charge returns the rest potential (v_reset, soft reset 0) exactly.
+__host__ __device__ inline bool cf_lif_silent_at_rest(const LifParams& p) {
+  return (p.hard ? p.v_reset : 0.0f) < p.v_th;
+}
+
 // Cache-policy operand of the raw buffer store builtins: the non-temporal
 // (streaming) hint.
 constexpr int CF_CPOL_NT = 2;

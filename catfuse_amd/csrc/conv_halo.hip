@@ -156,8 +156,8 @@ constexpr int halo_min_blocks() {
 // K: filter size (3, or 1 for pointwise convolutions, whose strided input
 // samples are staged densely: RH = TH, RW = TW).
 // LM: LIF specialisation (cf_lif_mode) of the EPI_LIF epilogue.
-// LEAN: the EPI_LIF epilogue without fp32 output or fp32 identity, every
-// output channel real (Cout a multiple of 64): no per-element branches.
+// LEAN: the EPI_LIF epilogue without fp32 output or fp32 identity: no
+// per-element branches.
 // ONEB: T fits one time block (T <= TB): the block loop runs once, so the
 // K-loop state is dead in the epilogue (fewer live registers).
 // HS: the SparseFlow route skips the MFMAs of a silent 16-channel chunk half
@@ -438,10 +438,10 @@ __device__ __forceinline__ void halo_body(const HaloArgs a, const int L, const i
           const int c = tid + 256 * i;
           const int px = c / CH8Z, part = c % CH8Z;
           const int py = px / TW, pxx = px % TW;
-          const bool ok = (oh0 + py < a.Ho) & (ow0 + pxx < a.Wo) & (cout0 + part * 8 < a.Cout);
+          const bool ok = (oh0 + py < a.Ho) & (ow0 + pxx < a.Wo) & (cout0 + part * 8 < a.cp_out);
           const int pix = (oh0 + py) * a.Wo + ow0 + pxx;
           const h8 sp = *reinterpret_cast<const h8*>(&srow[t * BM + part * 8]);
-          const uint32_t ioff = ok ? (uint32_t)((pix * a.cp_id + cout0 + part * 8) * XB) : HALO_OOB;
+          const uint32_t ioff = ok && cout0 + part * 8 < a.Cout ? (uint32_t)((pix * a.cp_id + cout0 + part * 8) * XB) : HALO_OOB;
           h8 idv;
           if constexpr (U8)
             idv = u8x8_to_h8(__builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(ri, ioff, 0, 0)));
@@ -1175,11 +1175,12 @@ __device__ __forceinline__ void halo_body(const HaloArgs a, const int L, const i
         const int c = tid + 256 * i;
         const int px = c / CH8, part = c % CH8;
         const int py = px / TW, pxx = px % TW;
-        const bool ok = (oh0 + py < a.Ho) & (ow0 + pxx < a.Wo) & (cout0 + part * 8 < a.Cout);
+        const bool ok = (oh0 + py < a.Ho) & (ow0 + pxx < a.Wo) & (cout0 + part * 8 < a.cp_out);
         const int pix = (oh0 + py) * a.Wo + ow0 + pxx;
         lo_off[i] = ok ? (uint32_t)((pix * a.cp_out + cout0 + part * 8) * XB) : HALO_OOB;
         lo_lds[i] = (uint32_t)(px * OLD + part * 8);
-        if constexpr (!U8) lo_id[i] = ok ? (uint32_t)((pix * a.cp_id + cout0 + part * 8) * 2) : HALO_OOB;
+        if constexpr (!U8)
+          lo_id[i] = ok && cout0 + part * 8 < a.Cout ? (uint32_t)((pix * a.cp_id + cout0 + part * 8) * 2) : HALO_OOB;
       }
     }
     // Lean fp16 path: the SEW identity is added to the staged tile at
@@ -1331,9 +1332,17 @@ hipError_t launch_halo(const HaloArgs& a, int epi, hipStream_t st) {
   // at most one workgroup per CU: the DEEP K loop (used where it exists)
   const int cus = cf_cu_count();
   const bool deep = cus > 0 && grid.x <= (unsigned)cus;
-  // lean: no fp32 output, no fp32 identity, whole 32-channel groups (the
-  // stores drop channels >= Cout of a partly real 64-channel tile)
-  const bool lean = epi == EPI_LIF && !a.out && !a.identity && a.Cout % 32 == 0;
+  // lean: no fp32 output, no fp32 identity; channels off 32 need a copy whose
+  // 16-byte chunks hold one pixel's channels (pitch a multiple of 8), an
+  // identity of the same pitch (zeros past Cout) and a neuron that stays silent
+  // without drive, so that the copy's channels past Cout (zero weights and
+  // BN coefficients) are zeros as they come.  Their general epilogue
+  // branches on every element, and its neuron on every parameter: 90 -> 170
+  // channels, 3x3 / 2 on 45 x 61, 5 images, 6 steps 68 -> 47 us.
+  const bool lean = epi == EPI_LIF && !a.out && !a.identity &&
+                    (a.Cout % 32 == 0 ||
+                     (a.cp_out % 8 == 0 && cf_lif_silent_at_rest(a.lif) &&
+                      (!a.identity_nhwc || a.cp_id == a.cp_out)));
   const bool oneb = a.T <= halo_tb<S, K>();
   if (a.u8) {
     // one-byte copies: the lean LIF epilogue on 8x8 tiles only (the SparseFlow

@@ -495,7 +495,7 @@ void conv_ring_kernel(const RingArgs a) {
 #pragma unroll
       for (int i = 0; i < CPI; ++i) {
         const int c = tid + 256 * i, pp = P0 + c / CH8, ch0 = cout0 + c % CH8 * 8;
-        const bool ok = pp < a.rows && ch0 < a.Cout;
+        const bool ok = pp < a.rows && ch0 < a.cp_out;
         co[i] = ok ? (uint32_t)((pp * a.cp_out + ch0) * 2) : HALO_OOB;
         ci[i] = ok ? (uint32_t)((pp * a.cp_id + ch0) * 2) : HALO_OOB;
       }
@@ -605,8 +605,9 @@ bool cf_conv_ring(int* rc, const void* x, const void* w_packed, const float* alp
                   int64_t Cout, int64_t Coutp, int64_t H, int64_t W, int64_t k, bool pool,
                   const LifParams& lif, hipStream_t st) {
   const int64_t rows = B * H * W, KK = k * k;
-  if (Cout % 32 != 0 || cp_out % 8 != 0 || (identity_nhwc && (cp_id % 8 != 0 || pool)))
-    return false;
+  if (cp_out % 8 != 0 || (identity_nhwc && (cp_id % 8 != 0 || cp_id < cp_out || pool)) ||
+      (Cout % 32 != 0 && (pool || !cf_lif_silent_at_rest(lif))))
+    return false;   // (channels past Cout are written as they come: zeros)
   if ((((uintptr_t)x | (uintptr_t)w_packed | (uintptr_t)out_nhwc | (uintptr_t)identity_nhwc) & 15))
     return false;
   if (T > 4 && !v_out) return false;
@@ -630,7 +631,7 @@ bool cf_conv_ring(int* rc, const void* x, const void* w_packed, const float* alp
   // What neighbouring workgroups share should be the larger operand.
   a.cb_major = 4 * Cout * KK * Cp > 8 * rows * Cp;
   const int64_t cus = cf_cu_count() > 0 ? cf_cu_count() : 256;
-  const int64_t n32 = a.ntiles * (Cout / 32), n64 = a.ntiles * (Coutp / 64);
+  const int64_t n32 = a.ntiles * ((Cout + 31) / 32), n64 = a.ntiles * (Coutp / 64);
   int mw = 1;
   if (k == 3) {
     // One workgroup per CU at a time (its LDS), so a launch takes whole
@@ -657,7 +658,7 @@ bool cf_conv_ring(int* rc, const void* x, const void* w_packed, const float* alp
     if (n32 > cus && n64 > cus) return false;
     mw = n32 <= cus ? 1 : 2;
   }
-  a.ncb = mw == 2 ? (int)(Coutp / 64) : (int)(Cout / 32);
+  a.ncb = mw == 2 ? (int)(Coutp / 64) : (int)((Cout + 31) / 32);
   if (nz_out && (unsigned long long)a.ntiles * a.ncb >= CF_MAX_COUNT_WG) return false;
   if (k == 3)
     *rc = (int)(W <= 14 ? launch_ring<3, 1, 96, 3, 9>(a, pool, st)

@@ -22,6 +22,8 @@ SHAPES = [
     (4, 1, 64, 64, 8, 8, 1), (4, 3, 96, 160, 14, 14, 1), (5, 1, 512, 64, 1, 1, 1),
     (2, 65, 300, 96, 1, 1, 1), (8, 4, 64, 64, 5, 7, 1), (1, 1, 32, 64, 3, 3, 1),
     (4, 30, 64, 704, 7, 7, 1),           # 64-channel tiles
+    (4, 2, 64, 70, 7, 7, 3), (5, 1, 32, 5, 9, 9, 3), (4, 2, 64, 37, 8, 8, 1),
+    (4, 30, 64, 690, 7, 7, 1),           # channels off 32 and off 64
 ]
 POOLED = [(4, 1, 64, 64, 16, 16), (4, 3, 96, 64, 8, 8), (6, 5, 64, 64, 4, 4),
           (4, 33, 64, 96, 2, 2), (3, 2, 32, 32, 6, 4), (1, 4, 512, 512, 2, 2)]
@@ -75,6 +77,7 @@ def test_flat_tiles(cuda, shape, ident, vin):
     xl = _lazy(x, cuda)
     idl = _lazy(i0, cuda) if ident else None
     y, v = r.run_mfma(xl, None if v0 is None else v0.to(cuda), identity=idl)
+    assert not bool(y._cf_nhwc[0][..., Co:].any())
     y, v = y.clone(), v.clone()
     ty, tv = _tiled(r, xl, None if v0 is None else v0.to(cuda), False,
                     idl._cf_nhwc[0] if ident else None)
@@ -112,3 +115,29 @@ def test_flat_tiles_zero_input(cuda, k, pool):
     y, v = r.run_mfma(x, epilogue=EPI_POOL if pool else EPI_LIF)
     ty, tv = _tiled(r, _lazy(x, cuda), None, pool, None)
     assert torch.equal(y.clone(), ty) and torch.equal(v.clone(), tv)
+
+
+@pytest.mark.parametrize("Co", [1, 31, 40, 70, 170])
+@pytest.mark.parametrize("k,stride,H,W,T,B", [(3, 1, 40, 33, 4, 3), (3, 2, 45, 61, 6, 2),
+                                              (1, 2, 31, 30, 4, 2), (3, 1, 35, 64, 9, 1)])
+@pytest.mark.parametrize("v_th", [0.3, -1.0])
+def test_channels_off_32(cuda, Co, k, stride, H, W, T, B, v_th):
+    """The lean epilogue of the 8x8-tile kernel at channel counts off 32: the
+    spikes, the sums with an identity and the state equal the general
+    epilogue's (fp32 output) bit for bit, and channels past Cout are zero in
+    the copy, also for a neuron that always fires."""
+    Ci = 48
+    g = torch.Generator().manual_seed(Co)
+    w = torch.randn(Co, Ci, k, k, generator=g) * (2.0 / (Co * k * k)) ** 0.5
+    r = ConvLIFRunner(w.to(cuda), None, None, None, stride, k // 2, 2.0, v_th, 0.0, True)
+    x = (torch.rand(T, B, Ci, H, W, generator=g) < 0.3).float()
+    Ho, Wo = r.out_hw(H, W)
+    i0 = torch.randint(0, 3, (T, B, Co, Ho, Wo), generator=g).float()
+    for ident in (None, i0):
+        for inp in (x, torch.zeros_like(x)):
+            xl = _lazy(inp, cuda)
+            y, v = r.run_mfma(xl, identity=None if ident is None else _lazy(ident, cuda))
+            assert not bool(y._cf_nhwc[0][..., Co:].any())
+            gy, gv = r.run_mfma(xl, identity=None if ident is None else ident.to(cuda),
+                                emit_nhwc=False)
+            assert torch.equal(y.clone(), gy) and torch.equal(v.clone(), gv)
