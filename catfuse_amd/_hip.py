@@ -30,6 +30,7 @@ _SIGNATURES = {
     "cf_pack_input": [_P, _I, _I, _I, _I, _I, _P, _P, c_int, c_float, _P, _P, _P],
     "cf_scan_nhwc": [_P, _I, _I, _I, _I, _I, _P, c_int, c_float, _P, _P],
     "cf_nhwc_to_nchw": [_P, _P, _I, _I, _I, _I, _I, _P],
+    "cf_copy_to_f32": [_P, _P, _P, _I, _I, _I, _I, _I, c_int, _P],
     "cf_global_avgpool_nhwc": [_P, _P, _P, _I, _I, _I, _I, _P],
     "cf_resolve_copy": [_P, _I, _P, _P],
     "cf_bias_response": [_P, _P, _I, _I, c_int, c_double, c_double, c_double, c_int, c_int, _P,

@@ -209,36 +209,67 @@ __global__ __launch_bounds__(256) void scan_nhwc_kernel(
 }
 
 // fp16 NHWC [NB][HW][cp] -> fp32 NCHW [NB][C][HW]: materialises the fp32
-// view of a fused conv output that was kept only as its NHWC copy.  A block
-// moves 64 pixels x 32 channels through LDS (reads: 64-byte runs per pixel;
-// writes: 256-byte runs per channel).
+// view of a fused conv output that was kept only as its NHWC copy, read where
+// its producer left it (desc, nullable: an all-zero copy gives zeros).  A
+// block moves 64 pixels x 64 channels through LDS, the reverse of
+// pack_kernel: a channel pair's halves are one word of a pixel's 33-word row;
+// reads are 128-byte runs per pixel, writes 16 bytes (four pixels of a channel)
+// a lane (128 images of 256 x 14 x 14 11.7 us, of 128 x 28 x 28 18.2; 4-byte
+// stores of 32-channel tiles took 12.5 and 17.6).  What reading through the
+// descriptor saves is the launch that filled unwritten copies first, 4.5 us of
+// the GPU's time and 5 of the host's.
 // XT: the copy's element, fp16 or one byte per channel (uint8_t).
 template <typename XT>
 __global__ __launch_bounds__(256) void nhwc_to_nchw_kernel(
-    const XT* __restrict__ xp, float* __restrict__ out, int64_t C, int64_t HW, int64_t cp) {
-  __shared__ float tile[CC][PX + 1];
+    const XT* __restrict__ xp_own, const CfOutDesc* __restrict__ desc, float* __restrict__ out,
+    int64_t C, int64_t HW, int64_t cp) {
+  typedef XT x8 __attribute__((ext_vector_type(8)));
+  typedef _Float16 h2 __attribute__((ext_vector_type(2)));
+  constexpr int TC = 64, LD = TC / 2 + 1;
+  __shared__ uint32_t tile[PX * LD];
   const int tid = threadIdx.x;
+  const XT* const xp = cf_copy_source(desc, xp_own);
   const int64_t n = blockIdx.z;
   const int64_t hw0 = (int64_t)blockIdx.x * PX;
-  const int64_t c0 = (int64_t)blockIdx.y * CC;
-  {
-    // read: 4 threads per pixel, 8 channels (16 or 8 bytes) each
-    const int px = tid / 4, part = tid % 4;
-    typedef XT x8 __attribute__((ext_vector_type(8)));
+  const int64_t c0 = (int64_t)blockIdx.y * TC;
+#pragma unroll
+  for (int i = 0; i < 2; ++i) {
+    // 8 threads per pixel, 8 channels (16 or 8 bytes) each
+    const int px = tid / 8 + 32 * i, part = tid % 8;
     x8 v = {};
-    if (hw0 + px < HW && c0 + part * 8 < cp)
+    if (xp != nullptr && hw0 + px < HW && c0 + part * 8 < cp)
       v = *reinterpret_cast<const x8*>(xp + ((n * HW + hw0 + px) * cp + c0 + part * 8));
 #pragma unroll
-    for (int j = 0; j < 8; ++j) tile[part * 8 + j][px] = (float)v[j];
+    for (int j = 0; j < 4; ++j) {
+      const h2 h = {(_Float16)v[2 * j], (_Float16)v[2 * j + 1]};   // bytes are exact in fp16
+      tile[px * LD + part * 4 + j] = __builtin_bit_cast(uint32_t, h);
+    }
   }
   __syncthreads();
-  // write: 64 consecutive pixels of one channel per 64 threads
-  const int px = tid % PX;
+  const int p0 = (tid % 16) * 4;
+  const int64_t left = HW - hw0 - p0;
 #pragma unroll
-  for (int i = 0; i < CC / 4; ++i) {
-    const int cl = tid / PX + 4 * i;
-    const int64_t c = c0 + cl;
-    if (c < C && hw0 + px < HW) out[(n * C + c) * HW + hw0 + px] = tile[cl][px];
+  for (int i = 0; i < 2; ++i) {
+    const int w = tid / 16 + 16 * i;
+    h2 h[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) h[j] = __builtin_bit_cast(h2, tile[(p0 + j) * LD + w]);
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int64_t c = c0 + 2 * w + u;
+      if (c >= C) continue;
+      float* dst = out + (n * C + c) * HW + hw0 + p0;
+      if (left >= 4) {
+        f32x4u q;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) q.v[j] = (float)h[j][u];
+        *reinterpret_cast<f32x4u*>(dst) = q;
+      } else {
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          if (j < left) dst[j] = (float)h[j][u];
+      }
+    }
   }
 }
 
@@ -360,7 +391,9 @@ __global__ __launch_bounds__(256) void pack_tokens_kernel(
 // load, two 16-byte stores): 25,088 rows of 384 20.6 -> 14.4 us against an
 // element a thread.
 __global__ __launch_bounds__(256) void tokens_to_f32_kernel(
-    const _Float16* __restrict__ xp, float* __restrict__ out, int64_t rows, int C, int cp) {
+    const _Float16* __restrict__ xp_own, const CfOutDesc* __restrict__ desc,
+    float* __restrict__ out, int64_t rows, int C, int cp) {
+  const _Float16* const xp = cf_copy_source(desc, xp_own);   // nullptr: all zero
   const uint32_t nc8 = (uint32_t)(C + 7) / 8u;
   const int64_t units = rows * nc8, step = (int64_t)gridDim.x * 256;
   const bool small = units + step < ((int64_t)1 << 32);   // 32-bit unit decode
@@ -373,7 +406,7 @@ __global__ __launch_bounds__(256) void tokens_to_f32_kernel(
     float* dst = out + r * C + c0;
     if (vec && c0 + 8 <= C) {
       typedef _Float16 h8 __attribute__((ext_vector_type(8)));
-      const h8 h = *reinterpret_cast<const h8*>(src);
+      const h8 h = xp != nullptr ? *reinterpret_cast<const h8*>(src) : h8{};
       f32x4u q0, q1;
 #pragma unroll
       for (int j = 0; j < 4; ++j) { q0.v[j] = (float)h[j]; q1.v[j] = (float)h[4 + j]; }
@@ -382,7 +415,7 @@ __global__ __launch_bounds__(256) void tokens_to_f32_kernel(
     } else {
 #pragma unroll
       for (int j = 0; j < 8; ++j)
-        if (c0 + j < C) dst[j] = (float)src[j];
+        if (c0 + j < C) dst[j] = xp != nullptr ? (float)src[j] : 0.0f;
     }
   }
 }
@@ -637,26 +670,48 @@ CF_API int cf_scan_nhwc(const void* xp, int64_t NB, int64_t H, int64_t W, int64_
 }
 
 template <typename XT>
-static int nhwc_to_nchw(const void* xp, float* out, int64_t NB, int64_t C, int64_t H, int64_t W,
-                        int64_t cp, void* stream) {
+static int nhwc_to_nchw(const void* xp, const void* desc, float* out, int64_t NB, int64_t C,
+                        int64_t H, int64_t W, int64_t cp, void* stream) {
   if (!xp || !out || NB < 0 || C <= 0 || H <= 0 || W <= 0 || cp < C || cp % 8 != 0 || NB > 65535)
     return (int)hipErrorInvalidValue;
   if (NB == 0) return 0;
   const int64_t HW = H * W;
-  dim3 grid(cf_blocks(HW, PX), (unsigned)((C + CC - 1) / CC), (unsigned)NB);
+  dim3 grid(cf_blocks(HW, PX), (unsigned)((C + 63) / 64), (unsigned)NB);
   hipLaunchKernelGGL(nhwc_to_nchw_kernel<XT>, grid, dim3(256), 0, (hipStream_t)stream,
-                     (const XT*)xp, out, C, HW, cp);
+                     (const XT*)xp, (const CfOutDesc*)desc, out, C, HW, cp);
   return (int)hipGetLastError();
+}
+
+static int tokens_to_f32(const void* xp, const void* desc, float* out, int64_t rows, int64_t C,
+                         int64_t cp, void* stream) {
+  if (!xp || !out || rows < 0 || C <= 0 || cp < C || rows * cp > ((int64_t)1 << 40))
+    return (int)hipErrorInvalidValue;
+  if (rows == 0) return 0;
+  const int64_t n = rows * ((C + 7) / 8);
+  const unsigned grid = (unsigned)((n + 255) / 256 < 16384 ? (n + 255) / 256 : 16384);
+  hipLaunchKernelGGL(tokens_to_f32_kernel, dim3(grid), dim3(256), 0, (hipStream_t)stream,
+                     (const _Float16*)xp, (const CfOutDesc*)desc, out, rows, (int)C, (int)cp);
+  return (int)hipGetLastError();
+}
+
+CF_API int cf_copy_to_f32(const void* xp, const void* desc, float* out, int64_t NB, int64_t C,
+                          int64_t H, int64_t W, int64_t cp, int tokens, void* stream) {
+  if (tokens != 0 && tokens != 1) return (int)hipErrorInvalidValue;
+  if (tokens) {
+    if (NB < 0 || H <= 0 || W <= 0) return (int)hipErrorInvalidValue;
+    return tokens_to_f32(xp, desc, out, NB * H * W, C, cp, stream);
+  }
+  return nhwc_to_nchw<_Float16>(xp, desc, out, NB, C, H, W, cp, stream);
 }
 
 CF_API int cf_nhwc_to_nchw(const void* xp, float* out, int64_t NB, int64_t C, int64_t H,
                            int64_t W, int64_t cp, void* stream) {
-  return nhwc_to_nchw<_Float16>(xp, out, NB, C, H, W, cp, stream);
+  return nhwc_to_nchw<_Float16>(xp, nullptr, out, NB, C, H, W, cp, stream);
 }
 
 CF_API int cf_nhwc_to_nchw_u8(const void* xp, float* out, int64_t NB, int64_t C, int64_t H,
                               int64_t W, int64_t cp, void* stream) {
-  return nhwc_to_nchw<uint8_t>(xp, out, NB, C, H, W, cp, stream);
+  return nhwc_to_nchw<uint8_t>(xp, nullptr, out, NB, C, H, W, cp, stream);
 }
 
 template <typename XT>
@@ -728,14 +783,7 @@ CF_API int cf_pack_tokens(const float* x, int64_t rows, int64_t C, int64_t cp, v
 
 CF_API int cf_tokens_to_f32(const void* xp, float* out, int64_t rows, int64_t C, int64_t cp,
                             void* stream) {
-  if (!xp || !out || rows < 0 || C <= 0 || cp < C || rows * cp > ((int64_t)1 << 40))
-    return (int)hipErrorInvalidValue;
-  if (rows == 0) return 0;
-  const int64_t n = rows * ((C + 7) / 8);
-  const unsigned grid = (unsigned)((n + 255) / 256 < 16384 ? (n + 255) / 256 : 16384);
-  hipLaunchKernelGGL(tokens_to_f32_kernel, dim3(grid), dim3(256), 0, (hipStream_t)stream,
-                     (const _Float16*)xp, out, rows, (int)C, (int)cp);
-  return (int)hipGetLastError();
+  return tokens_to_f32(xp, nullptr, out, rows, C, cp, stream);
 }
 
 CF_API int cf_linear_tokens(const void* xp, const void* desc, const float* w, const float* bias,

@@ -409,12 +409,12 @@ def _token_mean(args, kwargs) -> Optional[torch.Tensor]:
 class NHWCSpikes(_LazyTensor):
     """An fp32 NCHW [T, B, C, H, W] output of a fused layer whose values were
     written only as the fp16 NHWC copy the next fused layer reads.  The fp32
-    storage is filled (cf_nhwc_to_nchw) the first time anything other than a
+    storage is filled (cf_copy_to_f32) the first time anything other than a
     metadata query touches the tensor, so code outside the fused chain sees
     an ordinary tensor with the right values; fused layers that take the copy
     never pay for the fp32 form.  A copy its producer did not write (output
-    descriptor: all zero, or an alias of the identity's copy) is resolved
-    first (cf_resolve_copy)."""
+    descriptor: all zero, or an alias of the identity's copy) is read through
+    the descriptor (cf_copy_to_f32)."""
 
     @staticmethod
     def __new__(cls, base: torch.Tensor, nhwc: torch.Tensor, tokens: bool = False, meta=None):
@@ -433,22 +433,31 @@ class NHWCSpikes(_LazyTensor):
         self._cf_pending = False
         with torch._C.DisableTorchFunctionSubclass():
             nhwc = self._cf_nhwc[0]
-            _resolve(self, nhwc)
             cp = nhwc.shape[-1]
-            if nhwc.dtype == torch.uint8 and self.__dict__.get("_cf_tokens", False):
+            tokens = self.__dict__.get("_cf_tokens", False)
+            lib = _hip.lib()
+            if nhwc.dtype == torch.uint8:
+                _resolve(self, nhwc)
+                if not tokens:
+                    T, B, C, H, W = self.shape
+                    check(lib.cf_nhwc_to_nchw_u8(nhwc.data_ptr(), self.data_ptr(), T * B, C, H,
+                                                 W, cp, _hip.stream(self.device)),
+                          "cf_nhwc_to_nchw_u8")
+                    return
                 nhwc = _widen(self, nhwc)
-            if self.__dict__.get("_cf_tokens", False):
+            # one launch: the copy is read through its producer's descriptor
+            # (kept: the copy itself stays as it was left)
+            d = self.__dict__.get("_cf_desc")
+            if tokens:
                 # token-major [..., N, C]: a cast of the copy, dropping padding
                 C = self.shape[-1]
-                check(_hip.lib().cf_tokens_to_f32(nhwc.data_ptr(), self.data_ptr(),
-                                                  self.numel() // C, C, cp,
-                                                  _hip.stream(self.device)), "cf_tokens_to_f32")
-                return
-            T, B, C, H, W = self.shape
-            fn = (_hip.lib().cf_nhwc_to_nchw_u8 if nhwc.dtype == torch.uint8
-                  else _hip.lib().cf_nhwc_to_nchw)
-            check(fn(nhwc.data_ptr(), self.data_ptr(), T * B, C, H, W, cp,
-                     _hip.stream(self.device)), "cf_nhwc_to_nchw")
+                dims = (self.numel() // C, C, 1, 1)
+            else:
+                T, B, C, H, W = self.shape
+                dims = (T * B, C, H, W)
+            check(lib.cf_copy_to_f32(nhwc.data_ptr(), None if d is None else d[0].data_ptr(),
+                                     self.data_ptr(), *dims, cp, 1 if tokens else 0,
+                                     _hip.stream(self.device)), "cf_copy_to_f32")
 
 
 class ChannelState(_LazyTensor):

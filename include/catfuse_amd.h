@@ -112,6 +112,15 @@ int cf_scan_nhwc(const void* xp, int64_t NB, int64_t H, int64_t W, int64_t Cp, i
 int cf_nhwc_to_nchw(const void* xp, float* out, int64_t NB, int64_t C, int64_t H, int64_t W,
                     int64_t cp, void* stream);
 
+/* The fp32 form of a fused output whose fp16 copy xp is read through its
+ * output descriptor (desc, nullable: the copy is written; an all-zero copy
+ * gives zeros, an aliased one the values at the alias), so a copy its producer
+ * left unwritten need not be filled first.  tokens = 0: cf_nhwc_to_nchw of
+ * xp [NB][H][W][cp]; tokens = 1: token-major rows, out [NB*H*W][C].  No
+ * counterpart in the reference. */
+int cf_copy_to_f32(const void* xp, const void* desc, float* out, int64_t NB, int64_t C, int64_t H,
+                   int64_t W, int64_t cp, int tokens, void* stream);
+
 /* Global average pool of an fp16 NHWC copy xp [NB][HW][cp] (channels >= C
  * zero): out [NB][C] fp32 = (sum over the HW pixels) * float(1)/HW, which is
  * torch's GPU mean (AdaptiveAvgPool2d((1, 1)) = mean over H, W) bit for bit
