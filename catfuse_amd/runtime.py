@@ -1339,10 +1339,36 @@ class ConvLIFRunner:
                 out._cf_desc = (desc, base._version, keep)
         return out, v_out, nhwc, desc, info, v_chan
 
+    def _pack_record(self, x):
+        """(None, packing workspace, None, metadata) of a plain contiguous
+        fp32 GPU tensor x [T, B, Cin, H, W], in the place of a copy record
+        (_copy_record), or None: the inputs that run_mfma packs and nothing
+        else."""
+        if type(x) is not torch.Tensor or x.dtype != torch.float32 or not x.is_cuda:
+            return None
+        meta = _meta_of(x)
+        shape = meta[0]
+        if len(shape) != 5 or not meta[4] or shape[2] != self.Cin or shape[0] * shape[1] > 65535:
+            return None
+        xp = self.workspace("xp", (shape[0] * shape[1], shape[3], shape[4], self.Cp),
+                            torch.float16, meta[2])
+        return None, xp, None, meta
+
+    def _pack_planned(self, x, xp, shape, dev):
+        """pack_input of x into xp, as run_mfma calls it for a dense launch;
+        the layer's own count block."""
+        nnz = self.counter(dev)
+        check(_hip.lib().cf_pack_input(x.data_ptr(), shape[0] * shape[1], shape[2], shape[3],
+                                       shape[4], self.Cp, xp.data_ptr(), None, 0, 1e-6,
+                                       nnz.data_ptr(), status_word(dev).data_ptr(),
+                                       _hip.stream(dev)), "cf_pack_input")
+        return nnz
+
     def _dense_repeat(self, x, identity, want_v_out, sparse_threshold, epilogue=EPI_LIF):
         """run_mfma's launch for its common case from a plan cached per input
         signature: a dense-route LIF (or pooled LIF) launch with no initial
-        state whose input (and spike identity) carry a current NHWC copy,
+        state whose input (and spike identity) carry a current NHWC copy, or
+        whose input is a plain fp32 tensor (packed first, no identity),
         writing the output's copy, with no kernel timer.  The checks and
         choices that depend only on the signature (shapes, copy formats,
         device, whether the state is wanted, the copy settings) ran once when
@@ -1352,7 +1378,10 @@ class ConvLIFRunner:
         then takes its general path)."""
         rec = _copy_record(x)
         if rec is None:
-            return None
+            # a plain fp32 input is packed first (as run_mfma does)
+            rec = self._pack_record(x) if identity is None else None
+            if rec is None:
+                return None
         d, xp, ver, meta = rec
         xshape, dev = meta[0], meta[2]
         ish = None
@@ -1374,7 +1403,10 @@ class ConvLIFRunner:
                                                     epilogue)
         if p is False:
             return None
-        x_desc, nnz = _desc_count(d, ver)
+        if d is None:
+            x_desc, nnz = None, self._pack_planned(x, xp, xshape, dev)
+        else:
+            x_desc, nnz = _desc_count(d, ver)
         id_ptr = id_desc = id_nnz = 0
         id_keep = ()
         if identity is not None:
