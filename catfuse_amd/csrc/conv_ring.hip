@@ -90,10 +90,11 @@ struct RingGeom {
   static constexpr int DX = NX - 1, DW = NW - 1;  // slots a copy is issued ahead
   static constexpr int XL = XT / 1024;            // 1 KB copies of a step's pixels
   static constexpr int TW = 2 / MW, TPW = 2 * MW; // groups of time steps, steps a wave
+  static constexpr int NT = K == 3 ? 256 : 320;   // threads (1x1: a fifth wave copies weights)
 };
 
 template <int K, int MW, int NPX, int NX, int NW, int LM, bool POOL>
-__global__ __launch_bounds__(256, (RingGeom<K, MW, NPX, NX, NW>::LDS <= 80 * 1024 ? 2 : 1))
+__global__ __launch_bounds__((RingGeom<K, MW, NPX, NX, NW>::NT), 1)
 void conv_ring_kernel(const RingArgs a) {
   using G = RingGeom<K, MW, NPX, NX, NW>;
   constexpr int KK = G::KK, TB = G::TB, WB = G::WB, XT = G::XT, XB = G::XB, XL = G::XL;
@@ -104,7 +105,7 @@ void conv_ring_kernel(const RingArgs a) {
   static_assert(NPX % 16 == 0 && (K == 3 || NPX == 64), "staged pixels");
   __shared__ __attribute__((aligned(16))) char smem[G::LDS];
   __shared__ __attribute__((aligned(16))) float bn_s[2][BM];
-  __shared__ unsigned any_sh[4];
+  __shared__ unsigned any_sh[5];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -189,6 +190,45 @@ void conv_ring_kernel(const RingArgs a) {
     lds_buf_copy16_at(wr, voff, __builtin_amdgcn_readfirstlane(ch < nch ? so : 0u),
                       __builtin_amdgcn_readfirstlane(ring0 + slot * WB + f * 1024));
   };
+  // 1x1: the weights are wave 4's alone.  Loads complete in order, so a wave
+  // that waits for pixels (from the L2, where the layer before left them) would
+  // also wait for the weights it issued before them, which a network's pass
+  // brings from further away; a wave of their own keeps DW stages of them in
+  // flight (64 rows of 4096 -> 4096 38.3 -> 34.6 us; with 13 stages of weights
+  // but two pairs of pixels ahead instead of 5 and three, 39.8).  Its barriers
+  // are those of the other waves, one for one.
+  if constexpr (K == 1) {
+    if (wave == 4) {
+      for (int tb0 = 0; tb0 < a.T; tb0 += TB) {
+        if (!zero) {
+#pragma unroll
+          for (int s = 0; s < DW; ++s)
+#pragma unroll
+            for (int f = 0; f < 4 * MW; ++f) issue_w(f, s, 0, s);
+          wait_vm<(DW - 1) * 4 * MW>();
+          ring_barrier();
+          int wd = DW;
+          for (int ch = 0; ch < nch; ++ch) {
+            wait_vm<(DW - 2) * 4 * MW>();
+            ring_barrier();
+#pragma unroll
+            for (int f = 0; f < 4 * MW; ++f) issue_w(f, ch + DW, 0, wd);
+            wd = wd == NW - 1 ? 0 : wd + 1;
+          }
+        }
+        wait_vm<0>();
+        __syncthreads();
+        if (MW == 1) {      // the exchange of sums
+          __syncthreads();
+          __syncthreads();
+        }
+        __syncthreads();    // the staged output
+        if (tb0 + TB < a.T) __syncthreads();
+      }
+      if (a.nz_out != nullptr) cf_wg_any(false, any_sh);
+      return;
+    }
+  }
   // Pixel copy i of step `wave` of the block: 1 KB, 1024 / PB pixels.  A
   // pixel's 16-byte parts are stored in the order part ^ swizzle (3x3: pixel /
   // 4 % 4, 1x1: pixel / 2 % 8), which spreads the 16 lanes of a fragment read
@@ -367,46 +407,31 @@ void conv_ring_kernel(const RingArgs a) {
         }
       } else {
         // Stage s issues half (s % 2: pixels 0-31 or 32-63) of the chunk pair
-        // DX pairs ahead, then the weights of stage s + DW: PER copies a wave.
-        constexpr int XH = XL / 2, PER = XH + MW;
-        auto issue = [&](int c, int half, int pch, int pslot, int wch, int wslot) {
-          if (c < XH) issue_x(pch, half * XH + c, pslot);
-          else issue_w(wave * MW + c - XH, wch, 0, wslot);
-        };
-        constexpr int LEAD = DW > 2 * DX ? DW : 2 * DX;
+        // DX pairs ahead: XH copies a wave.
+        constexpr int XH = XL / 2;
 #pragma unroll
-        for (int s = -LEAD; s < 0; ++s)
-#pragma unroll
-          for (int c = 0; c < PER; ++c) {
-            // (pair (s + 2 DX) / 2 is chunks s + 2 DX and the next)
-            if (c < XH ? s + 2 * DX >= 0 : s + DW >= 0)
-              issue(c, s & 1, (s + 2 * DX) & ~1, (s + 2 * DX) / 2, s + DW, s + DW);
-          }
-        // What may be in flight once stage 0's copies have landed (weights of
-        // stage 0: issued DW stages ago; pair 0: its second half 2 DX - 1 ago).
-        constexpr int NP = MW + (2 * DX - 2) * PER, NQ = (DW - 1) * PER;
-        wait_vm<(NP < NQ || DW > 2 * DX) ? NP : NQ>();
+        for (int c = 0; c < DX * XL; ++c) issue_x(c / XL * 2, c % XL, c / XL);
+        wait_vm<(DX - 1) * XL>();                  // pair 0
         ring_barrier();
         read_frags(0, 0, 0, 0);
-        // ring slots: pair of stage ch + 1, pair being copied; weights of
-        // stages ch + 1 and ch + DW
-        int x1 = 0, xd = DX, w1 = 1 % NW, wd = DW;
+        // ring slots: pair of stage ch + 1, pair being copied, weights of
+        // stage ch + 1
+        int x1 = 0, xd = DX, w1 = 1 % NW;
         auto step = [&](auto set_c, int ch) {
           constexpr int odd = decltype(set_c)::v;   // ch % 2
-          // the next stage's weights, and after an odd one the next pair
-          constexpr int NWT = (DW - 2) * PER, NXT = MW + (2 * DX - 3) * PER;
           if (odd) x1 = x1 == NX - 1 ? 0 : x1 + 1;
           run_stage(
-              set_c, RingInt<PER>{},
+              set_c, RingInt<XH>{},
               [&] {
-                wait_vm<odd && NXT < NWT ? NXT : NWT>();
+                // an odd stage is followed by the next pair, whose second half
+                // was issued 2 DX - 2 stages ago
+                if (odd) wait_vm<(2 * DX - 3) * XH>();
                 ring_barrier();
               },
               [&] { return frag_src(w1, x1, odd ^ 1); },
-              [&](int c) { issue(c, odd, (ch & ~1) + 2 * DX, xd, ch + DW, wd); });
+              [&](int c) { issue_x((ch & ~1) + 2 * DX, odd * XH + c, xd); });
           if (odd) xd = xd == NX - 1 ? 0 : xd + 1;
           w1 = w1 == NW - 1 ? 0 : w1 + 1;
-          wd = wd == NW - 1 ? 0 : wd + 1;
         };
         for (int ch = 0; ch < nch; ch += 2) {
           step(RingInt<0>{}, ch);
@@ -571,7 +596,7 @@ void conv_ring_kernel(const RingArgs a) {
 
 template <int K, int MW, int NPX, int NX, int NW>
 hipError_t launch_ring(const RingArgs& a, bool pool, hipStream_t st) {
-  const dim3 grid((unsigned)(a.ntiles * a.ncb)), block(256);
+  const dim3 grid((unsigned)(a.ntiles * a.ncb)), block(RingGeom<K, MW, NPX, NX, NW>::NT);
 #define CF_RING(LMV, POOLV) \
   hipLaunchKernelGGL((conv_ring_kernel<K, MW, NPX, NX, NW, LMV, POOLV>), grid, block, 0, st, a)
   const int lm = cf_lif_mode(a.lif);
@@ -652,7 +677,7 @@ bool cf_conv_ring(int* rc, const void* x, const void* w_packed, const float* alp
     // another's loads in conv_halo.hip, which here waits for the LDS.
     // 32-channel tiles where they fit the round, else 64-channel ones.
     // Measured (us, 32 / 64 channels here / there, T = 4): 64 rows of 4096 ->
-    // 4096 37 / 51 / 87; 196 rows 1536 -> 384 18 / 25 / 34, 384 -> 1152 11 /
+    // 4096 35 / 51 / 87; 196 rows 1536 -> 384 18 / 25 / 34, 384 -> 1152 11 /
     // 14 / 15; 1,568 rows 1536 -> 384 36 (300 workgroups) / 26 / 39; 784 rows
     // 384 -> 1152 22 (468) / 16 / 20, 384 -> 1536 30 (624) / 28 (312) / 21.
     if (n32 > cus && n64 > cus) return false;
