@@ -76,9 +76,11 @@ __device__ __forceinline__ void ring_barrier() {
 
 // NPX: staged pixels of a step (3x3: at least 64 + 2 W + 3, the last one the
 // zero pixel; 1x1: 64).  NX: slots of the pixel ring, each the pixels of one
-// chunk (3x3: three) or of two (1x1: 128-byte runs of a pixel's channels, a
-// whole cache line, where a chunk alone is half of one).  NW: slots of the
-// weight ring (3x3: nine, a tap's slot is its number).
+// chunk (3x3: three, or two for layers of at most two chunks, which are then
+// both staged before the first tap: maps too wide for three slots) or of two
+// (1x1: 128-byte runs of a pixel's channels, a whole cache line, where a chunk
+// alone is half of one).  NW: slots of the weight ring (3x3: nine, a tap's slot
+// is its number).
 template <int K, int MW, int NPX, int NX, int NW>
 struct RingGeom {
   static constexpr int KK = K * K, TB = 4;
@@ -101,7 +103,8 @@ void conv_ring_kernel(const RingArgs a) {
   constexpr int DX = G::DX, DW = G::DW, PB = G::PB;
   constexpr int TPW = G::TPW, TW = G::TW, BM = 32 * MW;
   constexpr int NG = 4 / TW;                // groups of 4 channels a lane finishes
-  static_assert(K == 1 || (K == 3 && NX == 3 && NW == 9 && XL <= 9), "3x3: one slot a tap");
+  static_assert(K == 1 || (K == 3 && NW == 9 && (NX == 2 || (NX == 3 && XL <= 9))),
+                "3x3: one slot a tap");
   static_assert(NPX % 16 == 0 && (K == 3 || NPX == 64), "staged pixels");
   __shared__ __attribute__((aligned(16))) char smem[G::LDS];
   __shared__ __attribute__((aligned(16))) float bn_s[2][BM];
@@ -372,10 +375,10 @@ void conv_ring_kernel(const RingArgs a) {
           // after them may still be in flight (DW - 2 steps' copies).
           constexpr int nx = [] {
             int c = 0;
-            for (int k = 1; k <= DW - 2; ++k) c += (tap + 9 - k) % 9 < XL ? 1 : 0;
+            for (int k = 1; k <= DW - 2; ++k) c += NX == 3 && (tap + 9 - k) % 9 < XL ? 1 : 0;
             return c;
           }();
-          constexpr int XC = tap < XL ? 1 : 0;
+          constexpr int XC = NX == 3 && tap < XL ? 1 : 0;
           run_stage(
               set_c, RingInt<XC + MW>{},
               [&] {
@@ -399,7 +402,7 @@ void conv_ring_kernel(const RingArgs a) {
           step(RingInt<6>{}, RingInt<e>{}, ch); step(RingInt<7>{}, RingInt<o>{}, ch);
           step(RingInt<8>{}, RingInt<e>{}, ch);
           const int b = b0;
-          b0 = b1; b1 = b2; b2 = b;
+          b0 = b1; b1 = NX == 3 ? b2 : b; b2 = b;
         };
         for (int ch = 0; ch < nch; ch += 2) {
           chunk(RingInt<0>{}, ch);
@@ -601,7 +604,7 @@ hipError_t launch_ring(const RingArgs& a, bool pool, hipStream_t st) {
   hipLaunchKernelGGL((conv_ring_kernel<K, MW, NPX, NX, NW, LMV, POOLV>), grid, block, 0, st, a)
   const int lm = cf_lif_mode(a.lif);
   if (pool) {
-    if constexpr (K == 3) {
+    if constexpr (K == 3 && NX == 3) {             // (pooled maps are at most 16 wide)
       if (lm == LM_HARD0_DECAY_P2) CF_RING(LM_HARD0_DECAY_P2, true);
       else if (lm == LM_HARD_DECAY_P2) CF_RING(LM_HARD_DECAY_P2, true);
       else CF_RING(LM_GENERIC, true);
@@ -641,7 +644,7 @@ bool cf_conv_ring(int* rc, const void* x, const void* w_packed, const float* alp
   if (T * rows * Cout > INT32_MAX || 8 * rows * Cp > INT32_MAX || 4 * Coutp * KK * Cp > INT32_MAX ||
       rows * cp_out * 2 > INT32_MAX || rows * (identity_nhwc ? cp_id : 0) * 2 > INT32_MAX)
     return false;
-  if (k == 3 && W > 30) return false;
+  if (k == 3 && (W > 62 || (W > 30 && Cp > 2 * KC))) return false;
   if (pool && (k != 3 || !(W == 2 || W == 4 || W == 8 || W == 16) || H % 2 != 0)) return false;
   RingArgs a;
   a.x = (const _Float16*)x; a.w = (const _Float16*)w_packed; a.alpha = alpha; a.beta = beta;
@@ -666,7 +669,8 @@ bool cf_conv_ring(int* rc, const void* x, const void* w_packed, const float* alp
     // (us here / there, T = 4, SEW and VGG maps): 512 channels 7x7, 1 image
     // 27 / 54, 16 31 / 57, 32 (two rounds) 61 / 67; 4x4, 64 images 33 / 96;
     // 2x2, 64 27 / 91; 256 channels 14x14, 1 18 / 31, 8 21 / 34, 16 (two
-    // rounds) 39.4 / 38.7; 128 channels 28x28, 1 14 / 20, 8 (two) 28 / 23.
+    // rounds) 39.4 / 38.7; 128 channels 28x28, 1 14 / 20, 8 (two) 28 / 23; 64
+    // channels 56x56, 1 (two slots of pixels) 12.6 / 16.
     const int64_t stages = 9 * (Cp / KC);
     const int64_t halo_wg = B * ((H + 7) / 8) * ((W + 7) / 8) * (Coutp / 64);
     const int64_t here = (n32 + cus - 1) / cus * (9000 + 125 * stages);
@@ -686,8 +690,9 @@ bool cf_conv_ring(int* rc, const void* x, const void* w_packed, const float* alp
   a.ncb = mw == 2 ? (int)(Coutp / 64) : (int)((Cout + 31) / 32);
   if (nz_out && (unsigned long long)a.ntiles * a.ncb >= CF_MAX_COUNT_WG) return false;
   if (k == 3)
-    *rc = (int)(W <= 14 ? launch_ring<3, 1, 96, 3, 9>(a, pool, st)
-                        : launch_ring<3, 1, 128, 3, 9>(a, pool, st));
+    *rc = (int)(W <= 14   ? launch_ring<3, 1, 96, 3, 9>(a, pool, st)
+                : W <= 30 ? launch_ring<3, 1, 128, 3, 9>(a, pool, st)
+                          : launch_ring<3, 1, 192, 2, 9>(a, pool, st));
   else if (mw == 1)
     *rc = (int)launch_ring<1, 1, 64, 4, 6>(a, pool, st);
   else

@@ -21,6 +21,7 @@ SHAPES = [
     (1, 2, 64, 32, 1, 1, 3), (4, 17, 64, 64, 2, 2, 3), (9, 33, 33, 160, 3, 5, 3),
     (4, 1, 64, 64, 8, 8, 1), (4, 3, 96, 160, 14, 14, 1), (5, 1, 512, 64, 1, 1, 1),
     (2, 65, 300, 96, 1, 1, 1), (8, 4, 64, 64, 5, 7, 1), (1, 1, 32, 64, 3, 3, 1),
+    (4, 1, 64, 64, 56, 56, 3), (5, 2, 33, 32, 9, 62, 3), (4, 3, 32, 96, 5, 31, 3),  # two slots
     (4, 30, 64, 704, 7, 7, 1),           # 64-channel tiles
     (4, 2, 64, 70, 7, 7, 3), (5, 1, 32, 5, 9, 9, 3), (4, 2, 64, 37, 8, 8, 1),
     (4, 30, 64, 690, 7, 7, 1),           # channels off 32 and off 64
