@@ -377,6 +377,9 @@ __device__ __forceinline__ void halo_body(const HaloArgs a, const int L, const i
   // fewer than 2^31 elements).
   const int co_lane = cout0 + wm * WM + 4 * hi;
   const bool full_c = cout0 + BM <= a.Cout;  // every channel of the tile is real
+  // Lean stores: channels off 32 include the copy's padding (zeros, see the
+  // host's rule), whole groups end with the channels, whatever the copy's pitch.
+  const int c_end = (a.Cout & 31) == 0 ? a.Cout : a.cp_out;
 
   uint32_t anyw = 0u;  // OR of the bits of the output values this thread stores
   // The output's count block: workgroups that stored a nonzero value.
@@ -438,7 +441,7 @@ __device__ __forceinline__ void halo_body(const HaloArgs a, const int L, const i
           const int c = tid + 256 * i;
           const int px = c / CH8Z, part = c % CH8Z;
           const int py = px / TW, pxx = px % TW;
-          const bool ok = (oh0 + py < a.Ho) & (ow0 + pxx < a.Wo) & (cout0 + part * 8 < a.cp_out);
+          const bool ok = (oh0 + py < a.Ho) & (ow0 + pxx < a.Wo) & (cout0 + part * 8 < c_end);
           const int pix = (oh0 + py) * a.Wo + ow0 + pxx;
           const h8 sp = *reinterpret_cast<const h8*>(&srow[t * BM + part * 8]);
           const uint32_t ioff = ok && cout0 + part * 8 < a.Cout ? (uint32_t)((pix * a.cp_id + cout0 + part * 8) * XB) : HALO_OOB;
@@ -926,8 +929,8 @@ __device__ __forceinline__ void halo_body(const HaloArgs a, const int L, const i
     // 16-byte chunks, one 2*BM-byte run per pixel.  A spike-valued identity
     // (SEW ADD) is read from its fp16 NHWC copy when there is one: four
     // consecutive channels of a pixel per 8-byte load, exact for the integer
-    // values it holds.  The lean path (no fp32 output, no fp32 identity,
-    // every channel real) has no per-element branches: out-of-range pixels
+    // values it holds.  The lean path (no fp32 output, no fp32 identity) has
+    // no per-element branches: out-of-range pixels
     // are computed from zero halo and never stored.
     // The last taps' reads are complete, and so are the direct loads they
     // issued (zeros into the buffer the output is staged in below).
@@ -1111,7 +1114,9 @@ __device__ __forceinline__ void halo_body(const HaloArgs a, const int L, const i
           } else if constexpr (LEAN) {
             // (added at copy-out)
           } else {
-            if (idbase)
+            // (a 64-channel tile may reach past the copy's channels: at its last
+            // pixel that is past its memory)
+            if (idbase && col + 8 * r4 < a.cp_id)
               idh = *reinterpret_cast<const h4*>(idbase + (unsigned)(epix[nt] * a.cp_id + col + 8 * r4));
           }
           h4 pk;
@@ -1175,7 +1180,7 @@ __device__ __forceinline__ void halo_body(const HaloArgs a, const int L, const i
         const int c = tid + 256 * i;
         const int px = c / CH8, part = c % CH8;
         const int py = px / TW, pxx = px % TW;
-        const bool ok = (oh0 + py < a.Ho) & (ow0 + pxx < a.Wo) & (cout0 + part * 8 < a.cp_out);
+        const bool ok = (oh0 + py < a.Ho) & (ow0 + pxx < a.Wo) & (cout0 + part * 8 < c_end);
         const int pix = (oh0 + py) * a.Wo + ow0 + pxx;
         lo_off[i] = ok ? (uint32_t)((pix * a.cp_out + cout0 + part * 8) * XB) : HALO_OOB;
         lo_lds[i] = (uint32_t)(px * OLD + part * 8);

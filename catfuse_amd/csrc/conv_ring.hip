@@ -633,7 +633,7 @@ bool cf_conv_ring(int* rc, const void* x, const void* w_packed, const float* alp
                   int64_t Cout, int64_t Coutp, int64_t H, int64_t W, int64_t k, bool pool,
                   const LifParams& lif, hipStream_t st) {
   const int64_t rows = B * H * W, KK = k * k;
-  if (cp_out % 8 != 0 || (identity_nhwc && (cp_id % 8 != 0 || cp_id < cp_out || pool)) ||
+  if (cp_out != (Cout + 31) / 32 * 32 || (identity_nhwc && (cp_id % 8 != 0 || cp_id < cp_out || pool)) ||
       (Cout % 32 != 0 && (pool || !cf_lif_silent_at_rest(lif))))
     return false;   // (channels past Cout are written as they come: zeros)
   if ((((uintptr_t)x | (uintptr_t)w_packed | (uintptr_t)out_nhwc | (uintptr_t)identity_nhwc) & 15))
