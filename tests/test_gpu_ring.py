@@ -143,3 +143,30 @@ def test_channels_off_32(cuda, Co, k, stride, H, W, T, B, v_th):
             gy, gv = r.run_mfma(xl, identity=None if ident is None else ident.to(cuda),
                                 emit_nhwc=False)
             assert torch.equal(y.clone(), gy) and torch.equal(v.clone(), gv)
+
+
+@pytest.mark.parametrize("k,B,H", [(3, 1, 7), (1, 2, 8), (3, 3, 34)])
+def test_wide_copy_keeps_its_padding(cuda, k, B, H):
+    """An output copy whose pitch is wider than the channels need: channels
+    past Cout are left as they were, the others equal the usual pitch's."""
+    T, Ci, Co = 4, 64, 32
+    r = _layer(cuda, Ci, Co, k)[0]
+    dev = torch.device(cuda)
+    g = torch.Generator().manual_seed(3)
+    x = (torch.rand(T, B, Ci, H, H, generator=g) < 0.3).float().to(cuda)
+    r.run_mfma(x)                                    # (packs the weights)
+    xp = runtime.pack_input(x.reshape(T * B, Ci, H, H))[0]
+    p = runtime.ptr
+    outs = []
+    for cp in (32, 64):
+        out = torch.full((T * B, H, H, cp), 7.0, dtype=torch.float16, device=dev)
+        v = torch.empty((B, Co, H, H), device=dev)
+        rc = runtime._hip.lib().cf_conv_mfma(
+            p(xp), p(r.w_packed), p(r.alpha), p(r.beta), None, p(v), None, p(out), cp, None, None,
+            0, 1, None, None, None, None, None, None, None, 0, None, x.numel(), 2.0, T, B, r.Cp, Co,
+            r.Coutp, H, H, H, H, k, k, 1, k // 2, B, 0, 0, 0, EPI_LIF, *r.lif,
+            runtime._hip.stream(dev))
+        assert rc == 0
+        outs.append((out, v))
+    assert torch.equal(outs[0][0], outs[1][0][..., :Co]) and torch.equal(outs[0][1], outs[1][1])
+    assert bool((outs[1][0][..., Co:] == 7.0).all())
