@@ -71,3 +71,29 @@ def test_pack_flags_what_fp16_cannot_hold(cuda, where, bad):
         pack(x, status=st)
         # an infinity is an fp16 value; what rounds or is no number is not
         assert int(st) == (0 if bad == float("inf") else runtime.STATUS_INEXACT_FP16)
+
+
+@pytest.mark.parametrize("H,W,k,s,p", [(1, 1, 3, 2, 1), (7, 10, 3, 2, 1), (8, 9, 3, 2, 1),
+                                       (7, 10, 3, 1, 1)])
+def test_maxpool_order_with_nan(cuda, H, W, k, s, p):
+    """Where a copy holds NaN (an identity's), the pool's result is that of a
+    window walked by rows: its first value, and each later one that is greater
+    (a NaN is only kept in the first place), at the borders too."""
+    C = 40
+    g = torch.Generator().manual_seed(H)
+    v = torch.randint(0, 3, (2, 1, C, H, W), generator=g).float()
+    u = torch.rand(v.shape, generator=g)
+    v[u < 0.15], v[u > 0.9] = float("nan"), float("inf")
+    nhwc = torch.zeros(2, H, W, runtime.pad32(C), dtype=torch.float16)
+    nhwc[..., :C] = v.view(2, C, H, W).permute(0, 2, 3, 1).half()
+    y = runtime.maxpool_nhwc(runtime.lazy_output(tuple(v.shape), nhwc.to(cuda), cuda), k, s, p)
+    Ho, Wo = (H + 2 * p - k) // s + 1, (W + 2 * p - k) // s + 1
+    want = torch.empty(2, 1, C, Ho, Wo)
+    for oh in range(Ho):
+        for ow in range(Wo):
+            win = v[..., max(oh * s - p, 0):oh * s - p + k, max(ow * s - p, 0):ow * s - p + k]
+            m, *rest = win.flatten(3).unbind(3)
+            for q in rest:
+                m = torch.where(q > m, q, m)
+            want[..., oh, ow] = m
+    assert torch.equal(y.cpu().nan_to_num(7.0), want.nan_to_num(7.0))
