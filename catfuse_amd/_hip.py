@@ -96,6 +96,7 @@ _SIGNATURES = {
                        _I, _I, _I, c_int, c_double, c_double, c_double, c_int, c_int, _P],
     # argument blocks (ConvMfmaArgs / ConvHaloPairArgs below), by address
     "cf_conv_mfma_args": [_P],
+    "cf_conv_mfma_choice": [_P, _P],
     "cf_conv_halo_pair_args": [_P],
     "cf_conv_args_sizes": [_P],
 }

@@ -22,6 +22,35 @@ CF_ARGS_API int cf_conv_mfma_args(const CfConvMfmaArgs* a) {
                       (int)a->hard_reset, (int)a->decay_input, a->stream);
 }
 
+// conv_mfma.hip: cf_conv_mfma, or which kernel it would take.
+int cf_conv_mfma_run(const void* x, const void* w_packed, const float* alpha,
+                     const float* beta, const float* v_in, float* v_out, float* out,
+                     void* out_nhwc, int64_t cp_out,
+                     const float* identity, const void* identity_nhwc, int64_t cp_id,
+                     int identity_mode, const int32_t* ag_mask, const int32_t* tile_order,
+                     const unsigned long long* nnz, unsigned long long* nz_out,
+                     const void* x_desc, const void* id_desc, void* out_desc,
+                     int bias_info, const unsigned long long* id_nnz,
+                     int64_t numel, double sparse_threshold,
+                     int64_t T, int64_t B, int64_t Cp, int64_t Cout, int64_t Coutp, int64_t H,
+                     int64_t W, int64_t Ho, int64_t Wo, int64_t KH, int64_t KW, int64_t stride,
+                     int64_t pad, int64_t x_img_tstride, int64_t tile_h, int64_t tile_w,
+                     int64_t group_size, int epilogue, double tau, double v_th,
+                     double v_reset, int hard_reset, int decay_input, int* choice, void* stream);
+
+CF_ARGS_API int cf_conv_mfma_choice(const CfConvMfmaArgs* a, int* choice) {
+  if (!a || !choice) return (int)hipErrorInvalidValue;
+  return cf_conv_mfma_run(a->x, a->w_packed, a->alpha, a->beta, a->v_in, a->v_out, a->out,
+                          a->out_nhwc, a->cp_out, a->identity, a->identity_nhwc, a->cp_id,
+                          (int)a->identity_mode, a->ag_mask, a->tile_order, a->nnz, a->nz_out,
+                          a->x_desc, a->id_desc, a->out_desc, (int)a->bias_info, a->id_nnz,
+                          a->numel, a->sparse_threshold, a->T, a->B, a->Cp, a->Cout, a->Coutp,
+                          a->H, a->W, a->Ho, a->Wo, a->KH, a->KW, a->stride, a->pad,
+                          a->x_img_tstride, a->tile_h, a->tile_w, a->group_size,
+                          (int)a->epilogue, a->tau, a->v_th, a->v_reset, (int)a->hard_reset,
+                          (int)a->decay_input, choice, a->stream);
+}
+
 CF_ARGS_API int cf_conv_halo_pair_args(const CfConvHaloPairArgs* a) {
   if (!a) return (int)hipErrorInvalidValue;
   return cf_conv_halo_pair(a->x, a->nnz, a->x_desc, a->numel, a->T, a->B, a->Cp, a->H, a->W,

@@ -131,6 +131,9 @@ __host__ __device__ inline bool cf_lif_silent_at_rest(const LifParams& p) {
   return (p.hard ? p.v_reset : 0.0f) < p.v_th;
 }
 
+// The kernels a fused conv launch may take (CF_CONV_* of cf_conv_mfma_choice).
+enum { CONV_BY_GENERAL = 0, CONV_BY_HALO = 1, CONV_BY_HALO_LEAN = 2, CONV_BY_RING = 3 };
+
 // Cache-policy operand of the raw buffer store builtins: the non-temporal
 // (streaming) hint.
 constexpr int CF_CPOL_NT = 2;

@@ -1330,6 +1330,31 @@ void launch_lean(bool deep, dim3 grid, dim3 block, hipStream_t st, const HaloArg
                      st, a);
 }
 
+// One image's state and copies are addressed through 32-bit byte ranges in the
+// lean epilogue, and a lane with nothing to load or store takes the offset
+// HALO_OOB, which has to lie past each of them.  (The general epilogue's element
+// indices reach four times as far.)
+bool lean_ranges_ok(const HaloArgs& a) {
+  const int64_t HoWo = (int64_t)a.Ho * a.Wo, xb = a.u8 ? 1 : 2;
+  return (!a.v_out || HoWo * a.Cout * 4 <= INT32_MAX) && HoWo * a.cp_out * xb <= INT32_MAX &&
+         (!a.identity_nhwc || HoWo * a.cp_id * xb <= INT32_MAX);
+}
+
+// Whether a launch takes the lean epilogue: no fp32 output, no fp32 identity, an
+// image within its ranges; channels off 32 need a copy whose 16-byte chunks hold
+// one pixel's channels (pitch a multiple of 8), an identity of the same pitch
+// (zeros past Cout) and a neuron that stays silent without drive, so that the
+// copy's channels past Cout (zero weights and BN coefficients) are zeros as
+// they come.  Their general epilogue branches on every element, and its neuron
+// on every parameter: 90 -> 170 channels, 3x3 / 2 on 45 x 61, 5 images, 6 steps
+// 68 -> 47 us.
+bool halo_lean(const HaloArgs& a, int epi) {
+  return epi == EPI_LIF && !a.out && !a.identity && lean_ranges_ok(a) &&
+         (a.Cout % 32 == 0 ||
+          (a.cp_out % 8 == 0 && cf_lif_silent_at_rest(a.lif) &&
+           (!a.identity_nhwc || a.cp_id == a.cp_out)));
+}
+
 template <int TH, int TW, int S, int K = 3>
 hipError_t launch_halo(const HaloArgs& a, int epi, hipStream_t st) {
   dim3 grid((unsigned)(a.B * a.GH * a.GW * (a.Coutp / 64)));
@@ -1337,17 +1362,7 @@ hipError_t launch_halo(const HaloArgs& a, int epi, hipStream_t st) {
   // at most one workgroup per CU: the DEEP K loop (used where it exists)
   const int cus = cf_cu_count();
   const bool deep = cus > 0 && grid.x <= (unsigned)cus;
-  // lean: no fp32 output, no fp32 identity; channels off 32 need a copy whose
-  // 16-byte chunks hold one pixel's channels (pitch a multiple of 8), an
-  // identity of the same pitch (zeros past Cout) and a neuron that stays silent
-  // without drive, so that the copy's channels past Cout (zero weights and
-  // BN coefficients) are zeros as they come.  Their general epilogue
-  // branches on every element, and its neuron on every parameter: 90 -> 170
-  // channels, 3x3 / 2 on 45 x 61, 5 images, 6 steps 68 -> 47 us.
-  const bool lean = epi == EPI_LIF && !a.out && !a.identity &&
-                    (a.Cout % 32 == 0 ||
-                     (a.cp_out % 8 == 0 && cf_lif_silent_at_rest(a.lif) &&
-                      (!a.identity_nhwc || a.cp_id == a.cp_out)));
+  const bool lean = halo_lean(a, epi);
   const bool oneb = a.T <= halo_tb<S, K>();
   if (a.u8) {
     // one-byte copies: the lean LIF epilogue on 8x8 tiles only (the SparseFlow
@@ -1462,8 +1477,11 @@ int make_halo_args(HaloArgs& a, const void* x, const void* w_packed, const float
   // 32-channel groups, no identity (bias_info: the pooled bias response)
   if (epilogue == EPI_POOL &&
       (ksize != 3 || stride != 1 || tile_w != 8 || out || !out_nhwc || cp_out % 4 != 0 ||
-       Cout % 32 != 0 || identity || identity_nhwc || Ho < 2 || Wo < 2))
+       Cout % 32 != 0 || identity || identity_nhwc || Ho < 2 || Wo < 2 ||
+       (Ho / 2) * (Wo / 2) * cp_out * 2 > INT32_MAX))
     return (int)hipErrorInvalidValue;
+  // (its 32-bit byte range of the pooled state, Cout * (Ho / 2) * (Wo / 2) * 4,
+  // is within the bound on T * B * Cout * Ho * Wo below)
   if (!((tile_h == 8 && tile_w == 8) || (tile_h == 8 && tile_w == 16 && stride == 1 && ksize == 3)))
     return (int)hipErrorInvalidValue;
   if (ag_mask && (group_size <= 0 || (Cp + group_size - 1) / group_size > 32))
@@ -1587,8 +1605,9 @@ CF_API int cf_bias_response(const float* alpha, const float* beta, int64_t Cout,
 // 3x3 convolutions (stride 1 or 2, any padding) with halo staging; the
 // caller picks the tile (tile_h x tile_w in {8x8, 8x16}; 8x16 only with
 // stride 1).  u8: the copies (x, identity_nhwc, out_nhwc) hold one byte per
-// channel (8x8 tiles, lean LIF epilogue).
-static int conv_halo(const void* x, const void* w_packed, const float* alpha,
+// channel (8x8 tiles, lean LIF epilogue).  choice: not null, nothing is launched,
+// and *choice says whether the launch would take the lean epilogue.
+int cf_conv_halo_run(const void* x, const void* w_packed, const float* alpha,
                      const float* beta, const float* v_in, float* v_out, float* out,
                      void* out_nhwc, int64_t cp_out,
                      const float* identity, const void* identity_nhwc, int64_t cp_id,
@@ -1601,7 +1620,7 @@ static int conv_halo(const void* x, const void* w_packed, const float* alpha,
                      int64_t W, int64_t Ho, int64_t Wo, int64_t ksize, int64_t stride,
                      int64_t pad, int64_t tile_h, int64_t tile_w, int64_t group_size,
                      int epilogue, double tau, double v_th, double v_reset, int hard_reset,
-                     int decay_input, int u8, void* stream) {
+                     int decay_input, int u8, int* choice, void* stream) {
   HaloArgs a;
   const int rc = make_halo_args(a, x, w_packed, alpha, beta, v_in, v_out, out, out_nhwc, cp_out,
                                 identity, identity_nhwc, cp_id, identity_mode, ag_mask,
@@ -1616,6 +1635,10 @@ static int conv_halo(const void* x, const void* w_packed, const float* alpha,
              Cout % 32 != 0 || cp_out % 8 != 0 || Cp % 32 != 0))
     return (int)hipErrorInvalidValue;
   a.u8 = u8 ? 1 : 0;
+  if (choice != nullptr) {
+    *choice = halo_lean(a, epilogue) ? CONV_BY_HALO_LEAN : CONV_BY_HALO;
+    return 0;
+  }
   hipStream_t st = (hipStream_t)stream;
   hipError_t e;
   if (ksize == 1)
@@ -1643,11 +1666,12 @@ CF_API int cf_conv_halo(const void* x, const void* w_packed, const float* alpha,
                         int64_t pad, int64_t tile_h, int64_t tile_w, int64_t group_size,
                         int epilogue, double tau, double v_th, double v_reset, int hard_reset,
                         int decay_input, void* stream) {
-  return conv_halo(x, w_packed, alpha, beta, v_in, v_out, out, out_nhwc, cp_out, identity,
-                   identity_nhwc, cp_id, identity_mode, ag_mask, tile_order, nnz, nz_out, x_desc,
-                   id_desc, out_desc, bias_info, id_nnz, numel, sparse_threshold, T, B, Cp, Cout,
-                   Coutp, H, W, Ho, Wo, ksize, stride, pad, tile_h, tile_w, group_size, epilogue,
-                   tau, v_th, v_reset, hard_reset, decay_input, 0, stream);
+  return cf_conv_halo_run(x, w_packed, alpha, beta, v_in, v_out, out, out_nhwc, cp_out, identity,
+                          identity_nhwc, cp_id, identity_mode, ag_mask, tile_order, nnz, nz_out,
+                          x_desc, id_desc, out_desc, bias_info, id_nnz, numel, sparse_threshold,
+                          T, B, Cp, Cout, Coutp, H, W, Ho, Wo, ksize, stride, pad, tile_h, tile_w,
+                          group_size, epilogue, tau, v_th, v_reset, hard_reset, decay_input, 0,
+                          nullptr, stream);
 }
 
 CF_API int cf_conv_halo_u8(const void* x, const void* w_packed, const float* alpha,
@@ -1663,12 +1687,12 @@ CF_API int cf_conv_halo_u8(const void* x, const void* w_packed, const float* alp
                            int64_t stride, int64_t pad, int64_t group_size, double tau,
                            double v_th, double v_reset, int hard_reset, int decay_input,
                            void* stream) {
-  return conv_halo(x, w_packed, alpha, beta, v_in, v_out, nullptr, out_copy, cp_out, nullptr,
-                   identity_copy, cp_id, identity_copy ? ID_ADD_SPIKE : 0, ag_mask, tile_order,
-                   nnz, nz_out, x_desc, id_desc, out_desc, bias_info, id_nnz, numel,
-                   sparse_threshold, T, B, Cp, Cout, Coutp, H, W, Ho, Wo, ksize, stride, pad, 8,
-                   8, group_size, EPI_LIF, tau, v_th, v_reset, hard_reset, decay_input, 1,
-                   stream);
+  return cf_conv_halo_run(x, w_packed, alpha, beta, v_in, v_out, nullptr, out_copy, cp_out,
+                          nullptr, identity_copy, cp_id, identity_copy ? ID_ADD_SPIKE : 0, ag_mask,
+                          tile_order, nnz, nz_out, x_desc, id_desc, out_desc, bias_info, id_nnz,
+                          numel, sparse_threshold, T, B, Cp, Cout, Coutp, H, W, Ho, Wo, ksize,
+                          stride, pad, 8, 8, group_size, EPI_LIF, tau, v_th, v_reset, hard_reset,
+                          decay_input, 1, nullptr, stream);
 }
 
 static int conv_halo_pair(
@@ -1699,6 +1723,13 @@ static int conv_halo_pair(
                       v_reset, hard_reset, decay_input);
   if (rc) return rc;
   a.u8 = b.u8 = u8 ? 1 : 0;
+  if (!halo_lean(a, EPI_LIF) || !halo_lean(b, EPI_LIF)) {
+    // an image past the lean epilogue's ranges: two launches, each with the
+    // epilogue that covers it
+    if (u8) return (int)hipErrorInvalidValue;
+    const hipError_t e = launch_halo<8, 8, 2>(a, EPI_LIF, (hipStream_t)stream);
+    return (int)(e != hipSuccess ? e : launch_halo<8, 8, 2, 1>(b, EPI_LIF, (hipStream_t)stream));
+  }
   // each part's workgroup count as its own launch (below 2^23 together)
   const int64_t nLa = B * a.GH * a.GW * (Coutp_a / 64), nLb = B * b.GH * b.GW * (Coutp_b / 64);
   if (nLa + nLb >= ((int64_t)1 << 23)) return (int)hipErrorInvalidValue;

@@ -442,20 +442,21 @@ CF_API int cf_pack_conv_weights(const float* w, int64_t Cout, int64_t Cin, int64
   return (int)hipGetLastError();
 }
 
-CF_API int cf_conv_halo(const void* x, const void* w_packed, const float* alpha,
-                        const float* beta, const float* v_in, float* v_out, float* out,
-                        void* out_nhwc, int64_t cp_out,
-                        const float* identity, const void* identity_nhwc, int64_t cp_id,
-                        int identity_mode, const int32_t* ag_mask, const int32_t* tile_order,
-                        const unsigned long long* nnz, unsigned long long* nz_out,
-                        const void* x_desc, const void* id_desc, void* out_desc,
-                        int bias_info, const unsigned long long* id_nnz,
-                        int64_t numel, double sparse_threshold,
-                        int64_t T, int64_t B, int64_t Cp, int64_t Cout, int64_t Coutp, int64_t H,
-                        int64_t W, int64_t Ho, int64_t Wo, int64_t ksize, int64_t stride,
-                        int64_t pad, int64_t tile_h, int64_t tile_w, int64_t group_size,
-                        int epilogue, double tau, double v_th, double v_reset, int hard_reset,
-                        int decay_input, void* stream);
+// conv_halo.hip
+int cf_conv_halo_run(const void* x, const void* w_packed, const float* alpha,
+                     const float* beta, const float* v_in, float* v_out, float* out,
+                     void* out_nhwc, int64_t cp_out,
+                     const float* identity, const void* identity_nhwc, int64_t cp_id,
+                     int identity_mode, const int32_t* ag_mask, const int32_t* tile_order,
+                     const unsigned long long* nnz, unsigned long long* nz_out,
+                     const void* x_desc, const void* id_desc, void* out_desc,
+                     int bias_info, const unsigned long long* id_nnz,
+                     int64_t numel, double sparse_threshold,
+                     int64_t T, int64_t B, int64_t Cp, int64_t Cout, int64_t Coutp, int64_t H,
+                     int64_t W, int64_t Ho, int64_t Wo, int64_t ksize, int64_t stride,
+                     int64_t pad, int64_t tile_h, int64_t tile_w, int64_t group_size,
+                     int epilogue, double tau, double v_th, double v_reset, int hard_reset,
+                     int decay_input, int u8, int* choice, void* stream);
 
 // conv_ring.hip
 bool cf_conv_ring(int* rc, const void* x, const void* w_packed, const float* alpha,
@@ -465,28 +466,29 @@ bool cf_conv_ring(int* rc, const void* x, const void* w_packed, const float* alp
                   const void* id_desc, void* out_desc, int bias_info,
                   const unsigned long long* id_nnz, int64_t T, int64_t B, int64_t Cp,
                   int64_t Cout, int64_t Coutp, int64_t H, int64_t W, int64_t k, bool pool,
-                  const LifParams& lif, hipStream_t st);
+                  const LifParams& lif, bool launch, hipStream_t st);
 
-CF_API int cf_conv_mfma(const void* x, const void* w_packed, const float* alpha,
-                        const float* beta, const float* v_in, float* v_out, float* out,
-                        void* out_nhwc, int64_t cp_out,
-                        const float* identity, const void* identity_nhwc, int64_t cp_id,
-                        int identity_mode, const int32_t* ag_mask, const int32_t* tile_order,
-                        const unsigned long long* nnz, unsigned long long* nz_out,
-                        const void* x_desc, const void* id_desc, void* out_desc,
-                        int bias_info, const unsigned long long* id_nnz,
-                        int64_t numel, double sparse_threshold,
-                        int64_t T, int64_t B, int64_t Cp, int64_t Cout, int64_t Coutp, int64_t H,
-                        int64_t W, int64_t Ho, int64_t Wo, int64_t KH, int64_t KW, int64_t stride,
-                        int64_t pad, int64_t x_img_tstride, int64_t tile_h, int64_t tile_w,
-                        int64_t group_size, int epilogue, double tau, double v_th,
-                        double v_reset, int hard_reset, int decay_input, void* stream) {
+// cf_conv_mfma; with choice not null nothing is launched, and *choice says which
+// kernel the launch would take (CF_CONV_*).
+int cf_conv_mfma_run(const void* x, const void* w_packed, const float* alpha,
+                     const float* beta, const float* v_in, float* v_out, float* out,
+                     void* out_nhwc, int64_t cp_out,
+                     const float* identity, const void* identity_nhwc, int64_t cp_id,
+                     int identity_mode, const int32_t* ag_mask, const int32_t* tile_order,
+                     const unsigned long long* nnz, unsigned long long* nz_out,
+                     const void* x_desc, const void* id_desc, void* out_desc,
+                     int bias_info, const unsigned long long* id_nnz,
+                     int64_t numel, double sparse_threshold,
+                     int64_t T, int64_t B, int64_t Cp, int64_t Cout, int64_t Coutp, int64_t H,
+                     int64_t W, int64_t Ho, int64_t Wo, int64_t KH, int64_t KW, int64_t stride,
+                     int64_t pad, int64_t x_img_tstride, int64_t tile_h, int64_t tile_w,
+                     int64_t group_size, int epilogue, double tau, double v_th,
+                     double v_reset, int hard_reset, int decay_input, int* choice, void* stream) {
   if (!x || !w_packed || !alpha || !beta || (!out && !out_nhwc)) return (int)hipErrorInvalidValue;
   if (T <= 0 || B <= 0 || Cp <= 0 || Cp % KC != 0 || Cout <= 0 || Coutp < Cout ||
       Coutp % 64 != 0 || H <= 0 || W <= 0 || Ho <= 0 || Wo <= 0 || KH <= 0 || KW <= 0 ||
       stride <= 0 || pad < 0 || x_img_tstride < 0)
     return (int)hipErrorInvalidValue;
-  // EPI_POOL (BN -> AvgPool2d(2, 2) -> LIF) runs in the halo kernel only
   if (epilogue != EPI_LIF && epilogue != EPI_Z && epilogue != EPI_POOL)
     return (int)hipErrorInvalidValue;
   if (identity && identity_mode != ID_ADD_SPIKE && identity_mode != ID_ADD_Z)
@@ -500,10 +502,11 @@ CF_API int cf_conv_mfma(const void* x, const void* w_packed, const float* alpha,
     return (int)hipErrorInvalidValue;
   const bool rect = tile_h > 0 && tile_w > 0;
   // 3x3 convolutions and 1x1 convolutions over feature maps of at least
-  // 4x4 (stride 1/2, pad <= 2, one time-major input) always take the
-  // halo-staged kernel, whatever the route or epilogue, so every
-  // implementation of a layer accumulates in the same order.  The choice
-  // depends on the layer shape only.
+  // 4x4 (stride 1/2, pad <= 2, one time-major input) take the halo-staged
+  // kernel, whatever the route or epilogue, or the flat-tile kernel below.
+  // Both accumulate in the same order, which so depends on the layer's shape
+  // only: every implementation of a layer gives the same bits.  EPI_POOL (BN ->
+  // AvgPool2d(2, 2) -> LIF) runs in these two only.
   const bool k_ok = (KH == 3 && KW == 3) || (KH == 1 && KW == 1 && Ho >= 4 && Wo >= 4);
   const bool halo_ok = k_ok && (stride == 1 || stride == 2) && pad <= 2 &&
                        x_img_tstride == B && T * B * Cout * Ho * Wo <= INT32_MAX &&
@@ -521,17 +524,20 @@ CF_API int cf_conv_mfma(const void* x, const void* w_packed, const float* alpha,
                      cp_id, nnz, nz_out, x_desc, id_desc, out_desc, bias_info, id_nnz, T, B, Cp,
                      Cout, Coutp, H, W, KH, epilogue == EPI_POOL,
                      cf_make_lif_params(tau, v_th, v_reset, hard_reset, decay_input),
-                     (hipStream_t)stream))
+                     choice == nullptr, (hipStream_t)stream)) {
+      if (choice != nullptr) *choice = CONV_BY_RING;
       return rc;
+    }
   }
   if (halo_ok) {
     const int64_t th = 8, tw = rect ? tile_w : 8;
-    return cf_conv_halo(x, w_packed, alpha, beta, v_in, v_out, out, out_nhwc, cp_out, identity,
-                        identity_nhwc, cp_id, identity_mode,
-                        rect ? ag_mask : nullptr, rect ? tile_order : nullptr, nnz, nz_out,
-                        x_desc, id_desc, out_desc, bias_info, id_nnz, numel, sparse_threshold, T, B, Cp, Cout,
-                        Coutp, H, W, Ho, Wo, KH, stride, pad, th, tw, rect ? group_size : 0,
-                        epilogue, tau, v_th, v_reset, hard_reset, decay_input, stream);
+    return cf_conv_halo_run(x, w_packed, alpha, beta, v_in, v_out, out, out_nhwc, cp_out, identity,
+                            identity_nhwc, cp_id, identity_mode,
+                            rect ? ag_mask : nullptr, rect ? tile_order : nullptr, nnz, nz_out,
+                            x_desc, id_desc, out_desc, bias_info, id_nnz, numel, sparse_threshold,
+                            T, B, Cp, Cout, Coutp, H, W, Ho, Wo, KH, stride, pad, th, tw,
+                            rect ? group_size : 0, epilogue, tau, v_th, v_reset, hard_reset,
+                            decay_input, 0, choice, stream);
   }
   if (rect) {
     if (!(tile_h * tile_w == 64 || tile_h * tile_w == 128)) return (int)hipErrorInvalidValue;
@@ -574,6 +580,10 @@ CF_API int cf_conv_mfma(const void* x, const void* w_packed, const float* alpha,
   if (nz_out && (unsigned long long)n_ptiles * (Coutp / 64) >= CF_MAX_COUNT_WG)
     return (int)hipErrorInvalidValue;
   a.n_ptiles = n_ptiles;
+  if (choice != nullptr) {
+    *choice = CONV_BY_GENERAL;
+    return 0;
+  }
   hipStream_t st = (hipStream_t)stream;
   hipError_t e;
   if (rect) e = epilogue == EPI_Z ? pick_tiles<true, EPI_Z>(a, BMsel, BNsel, n_ptiles, st)
@@ -581,4 +591,26 @@ CF_API int cf_conv_mfma(const void* x, const void* w_packed, const float* alpha,
   else e = epilogue == EPI_Z ? pick_tiles<false, EPI_Z>(a, BMsel, BNsel, n_ptiles, st)
                              : pick_tiles<false, EPI_LIF>(a, BMsel, BNsel, n_ptiles, st);
   return (int)e;
+}
+
+CF_API int cf_conv_mfma(const void* x, const void* w_packed, const float* alpha,
+                        const float* beta, const float* v_in, float* v_out, float* out,
+                        void* out_nhwc, int64_t cp_out,
+                        const float* identity, const void* identity_nhwc, int64_t cp_id,
+                        int identity_mode, const int32_t* ag_mask, const int32_t* tile_order,
+                        const unsigned long long* nnz, unsigned long long* nz_out,
+                        const void* x_desc, const void* id_desc, void* out_desc,
+                        int bias_info, const unsigned long long* id_nnz,
+                        int64_t numel, double sparse_threshold,
+                        int64_t T, int64_t B, int64_t Cp, int64_t Cout, int64_t Coutp, int64_t H,
+                        int64_t W, int64_t Ho, int64_t Wo, int64_t KH, int64_t KW, int64_t stride,
+                        int64_t pad, int64_t x_img_tstride, int64_t tile_h, int64_t tile_w,
+                        int64_t group_size, int epilogue, double tau, double v_th,
+                        double v_reset, int hard_reset, int decay_input, void* stream) {
+  return cf_conv_mfma_run(x, w_packed, alpha, beta, v_in, v_out, out, out_nhwc, cp_out, identity,
+                          identity_nhwc, cp_id, identity_mode, ag_mask, tile_order, nnz, nz_out,
+                          x_desc, id_desc, out_desc, bias_info, id_nnz, numel, sparse_threshold,
+                          T, B, Cp, Cout, Coutp, H, W, Ho, Wo, KH, KW, stride, pad, x_img_tstride,
+                          tile_h, tile_w, group_size, epilogue, tau, v_th, v_reset, hard_reset,
+                          decay_input, nullptr, stream);
 }

@@ -622,8 +622,8 @@ hipError_t launch_ring(const RingArgs& a, bool pool, hipStream_t st) {
 
 // Runs one conv of the cf_conv_mfma argument list here when this kernel
 // covers it and is the faster one; returns false (nothing launched) otherwise,
-// else sets *rc.  (Called with the arguments cf_conv_mfma has checked, no
-// tile masks.)
+// else sets *rc (launch false: only says which).  (Called with the arguments
+// cf_conv_mfma has checked, no tile masks.)
 bool cf_conv_ring(int* rc, const void* x, const void* w_packed, const float* alpha,
                   const float* beta, const float* v_in, float* v_out, void* out_nhwc,
                   int64_t cp_out, const void* identity_nhwc, int64_t cp_id,
@@ -631,7 +631,7 @@ bool cf_conv_ring(int* rc, const void* x, const void* w_packed, const float* alp
                   const void* id_desc, void* out_desc, int bias_info,
                   const unsigned long long* id_nnz, int64_t T, int64_t B, int64_t Cp,
                   int64_t Cout, int64_t Coutp, int64_t H, int64_t W, int64_t k, bool pool,
-                  const LifParams& lif, hipStream_t st) {
+                  const LifParams& lif, bool launch, hipStream_t st) {
   const int64_t rows = B * H * W, KK = k * k;
   if (cp_out != (Cout + 31) / 32 * 32 || (identity_nhwc && (cp_id % 8 != 0 || cp_id < cp_out || pool)) ||
       (Cout % 32 != 0 && (pool || !cf_lif_silent_at_rest(lif))))
@@ -689,6 +689,7 @@ bool cf_conv_ring(int* rc, const void* x, const void* w_packed, const float* alp
   }
   a.ncb = mw == 2 ? (int)(Coutp / 64) : (int)((Cout + 31) / 32);
   if (nz_out && (unsigned long long)a.ntiles * a.ncb >= CF_MAX_COUNT_WG) return false;
+  if (!launch) return true;
   if (k == 3)
     *rc = (int)(W <= 14   ? launch_ring<3, 1, 96, 3, 9>(a, pool, st)
                 : W <= 30 ? launch_ring<3, 1, 128, 3, 9>(a, pool, st)

@@ -1207,12 +1207,14 @@ class ConvLIFRunner:
 
     def halo_lean_ok(self, T, B, Ho, Wo) -> bool:
         """Whether a launch of this layer at output size Ho x Wo runs the
-        halo kernel (3x3, or 1x1 over maps of at least 4x4; stride 1 or 2),
+        halo kernel with its lean epilogue (3x3, or 1x1 over maps of at least
+        4x4; stride 1 or 2; one image's state within a 31-bit byte range),
         which the byte-copy path needs."""
         k_ok = ((self.KH, self.KW) == (3, 3)
                 or ((self.KH, self.KW) == (1, 1) and Ho >= 4 and Wo >= 4))
         return (k_ok and self.stride in (1, 2) and self.padding <= 2
-                and T * B * self.Cout * Ho * Wo <= 2 ** 31 - 1)
+                and T * B * self.Cout * Ho * Wo <= 2 ** 31 - 1
+                and 4 * self.Cout * Ho * Wo <= 2 ** 31 - 1)
 
     def out_hw(self, H, W):
         return ((H + 2 * self.padding - self.KH) // self.stride + 1,
@@ -2126,10 +2128,11 @@ def _halo_pair_plan(ra, rb, x, xp, meta):
         return False
     if xp.device != dev or tuple(xp.shape) != (T * B, H, W, ra.Cp):
         return False
-    u8 = SPIKE_COPY == "u8" and xp.dtype == torch.uint8
+    Ho, Wo = ra.out_hw(H, W)
+    u8 = (SPIKE_COPY == "u8" and xp.dtype == torch.uint8
+          and ra.halo_lean_ok(T, B, Ho, Wo) and rb.halo_lean_ok(T, B, Ho, Wo))
     if xp.dtype != (torch.uint8 if u8 else torch.float16):
         return False
-    Ho, Wo = ra.out_hw(H, W)
     p = _PairPlan()
     p.rb, p.rb_key = rb, rb._packed_key
     p.u8 = u8
@@ -2253,7 +2256,8 @@ def run_halo_pair(ra: "ConvLIFRunner", rb: "ConvLIFRunner", x: torch.Tensor, v_i
     Ho, Wo = ra.out_hw(H, W)
     # byte copies in, byte copies out (cf_conv_halo_pair_u8)
     cand = (shadow_of(x, (T * B, H, W, ra.Cp), resolve=False, u8_ok=True)
-            if SPIKE_COPY == "u8" else None)
+            if (SPIKE_COPY == "u8" and ra.halo_lean_ok(T, B, Ho, Wo)
+                and rb.halo_lean_ok(T, B, Ho, Wo)) else None)
     u8 = cand is not None and cand.dtype == torch.uint8
     xp = shadow_of(x, (T * B, H, W, ra.Cp), resolve=False, u8_ok=u8)
     x_desc = None

@@ -354,7 +354,7 @@ int cf_pack_conv_weights(const float* w, int64_t Cout, int64_t Cin, int64_t KH, 
  *   launch writes its outputs and records so.  A caller that passes
  *   out_desc reads the outputs through it (or hands it on as x_desc /
  *   id_desc).
- *   Epilogue 2 (stride-1 3x3 convs on 8x8 tiles, the halo kernel): each 2x2
+ *   Epilogue 2 (stride-1 3x3 convs on 8x8 tiles or flat ones): each 2x2
  *   window of BN outputs is summed as ((z00 + z01) + z10) + z11, times
  *   0.25 (the order of cf_avgpool2x2_lif, so the spikes equal epilogue 1
  *   followed by cf_avgpool2x2_lif bit for bit), and drives the pooled
@@ -540,6 +540,12 @@ typedef struct CfConvHaloPairArgs {
 } CfConvHaloPairArgs;
 
 int cf_conv_mfma_args(const CfConvMfmaArgs* args);
+/* Which kernel cf_conv_mfma_args(args) launches, without launching it: the
+ * general kernel, the halo kernel with its general or its lean epilogue, or the
+ * flat-tile kernel (all give the same bits).  Takes what the launch takes, and
+ * returns its error for what it refuses.  No counterpart in the reference. */
+enum { CF_CONV_GENERAL = 0, CF_CONV_HALO = 1, CF_CONV_HALO_LEAN = 2, CF_CONV_RING = 3 };
+int cf_conv_mfma_choice(const CfConvMfmaArgs* args, int* choice);
 int cf_conv_halo_pair_args(const CfConvHaloPairArgs* args);
 int cf_conv_args_sizes(int64_t* sizes);
 
@@ -557,8 +563,10 @@ int cf_conv_args_sizes(int64_t* sizes);
  * cf_conv_halo_u8: cf_conv_halo with the lean LIF epilogue (no fp32 output,
  * identity only as a copy: identity_copy nullable, added to the spikes),
  * 8x8 tiles, Cout a multiple of 32, cp_out a multiple of 8, Cp of 32;
- * x / identity_copy / out_copy one byte per channel; other arguments as
- * cf_conv_halo.  cf_conv_halo_pair_u8: cf_conv_halo_pair on byte copies.
+ * x / identity_copy / out_copy one byte per channel; one image's state
+ * (when v_out is given) and copies below 2^31 bytes (cf_conv_halo's general
+ * epilogue takes fp16 copies past that); other arguments as cf_conv_halo.
+ * cf_conv_halo_pair_u8: cf_conv_halo_pair on byte copies.
  * cf_conv_stem_lif_maxpool_u8: the stem writing its pooled output as a byte
  * copy (out_copy).  cf_nhwc_to_nchw_u8 / cf_global_avgpool_nhwc_u8: as the
  * fp16 forms, reading a byte copy.  cf_copy_u8_to_f16: a byte copy of n

@@ -246,3 +246,76 @@ def test_argument_block_entry_points_reject_null():
     assert _hip.lib().cf_conv_mfma_args(None) == INVALID
     assert _hip.lib().cf_conv_halo_pair_args(None) == INVALID
     assert _hip.lib().cf_conv_args_sizes(None) == INVALID
+
+
+def test_lean_epilogue_stays_within_its_byte_ranges():
+    """The halo kernel's lean epilogue addresses one image's state and copies
+    through 32-bit byte ranges whose masked lanes take offset 2^31: an image
+    past 2^31 - 1 bytes of either takes the general epilogue, whatever its
+    channels."""
+    from choice import HALO, HALO_LEAN, conv_choice
+    for Co in (100, 170, 128, 192):
+        for n in (1500, 1700, 2000, 2300, 2400):
+            state, copy = 4 * Co * n * n, 2 * runtime_pad32(Co) * n * n
+            want = HALO_LEAN if max(state, copy) < 2 ** 31 else HALO
+            assert conv_choice(1, 1, 32, Co, n, n, 3) == want, (Co, n)
+            want = HALO_LEAN if copy < 2 ** 31 else HALO
+            assert conv_choice(1, 1, 32, Co, n, n, 3, state=False) == want, (Co, n)
+    assert conv_choice(1, 1, 32, 128, 2048, 2047, 3) == HALO_LEAN
+    assert conv_choice(1, 1, 32, 128, 2048, 2048, 3) == HALO
+    assert conv_choice(1, 1, 32, 100, 2888, 2888, 3, stride=2) == HALO_LEAN
+    assert conv_choice(1, 1, 32, 300, 2888, 2888, 3, stride=2) == HALO
+    # an identity copy of wider pitch, its own range
+    assert conv_choice(1, 1, 32, 64, 2000, 2000, 3, ident=True, cp_id=128) == HALO_LEAN
+    assert conv_choice(1, 1, 32, 64, 2000, 2000, 3, ident=True, cp_id=512) == HALO
+    # pooled copies have no other epilogue: refused
+    assert conv_choice(1, 1, 32, 32, 2000, 2000, 3, pool=True, cp_out=1024) == HALO
+    assert conv_choice(1, 1, 32, 32, 2048, 2048, 3, pool=True, cp_out=1024) is None
+
+
+def runtime_pad32(c):
+    from catfuse_amd import runtime
+    return runtime.pad32(c)
+
+
+def test_byte_copies_past_the_lean_ranges():
+    """The one-byte entry points have the lean epilogue only: images past its
+    ranges are refused, and the runtime widens such layers' copies."""
+    import torch
+    from catfuse_amd import _hip, runtime
+    L = _hip.lib()
+
+    def halo_u8(n, Co=128):
+        return L.cf_conv_halo_u8(1, 1, 1, 1, None, 1, 1, Co, None, Co, None, None, None, None,
+                                 None, None, None, 0, None, 0, 2.0, 1, 1, 32, Co, Co, n, n, n, n,
+                                 3, 1, 1, 0, 2.0, 1.0, 0.0, 1, 1, None)
+
+    def pair_u8(n, Co=320):
+        h = n // 2
+        return L.cf_conv_halo_pair_u8(1, None, None, 0, 1, 1, 32, n, n, h, h,
+                                      1, 1, 1, None, 1, 1, 64, None, None, 0, 64, 64, 1,
+                                      1, 1, 1, None, 1, 1, Co, None, None, 0, Co, Co, 0,
+                                      2.0, 1.0, 0.0, 1, 1, None)
+    assert halo_u8(2400) == INVALID
+    assert pair_u8(2888) == INVALID
+    r = runtime.ConvLIFRunner(torch.zeros(128, 32, 3, 3), None, None, None, 1, 1, 2.0, 1.0, 0.0,
+                              True)
+    assert r.halo_lean_ok(1, 1, 2048, 2047) and not r.halo_lean_ok(1, 1, 2048, 2048)
+
+
+def test_flat_tile_kernel_bounds():
+    """Where cf_conv_mfma leaves the flat-tile kernel: maps too wide for its
+    staged pixels, copies of another pitch, outputs it does not write."""
+    from choice import GENERAL, HALO, HALO_LEAN, RING, conv_choice
+    assert conv_choice(4, 1, 64, 64, 5, 62, 3) == RING
+    assert conv_choice(4, 1, 64, 64, 5, 63, 3) == HALO_LEAN
+    assert conv_choice(4, 1, 96, 64, 5, 30, 3) == RING
+    assert conv_choice(4, 1, 96, 64, 5, 31, 3) == HALO_LEAN
+    assert conv_choice(4, 1, 64, 64, 7, 7, 3, cp_out=128) == HALO_LEAN
+    assert conv_choice(4, 1, 64, 64, 8, 8, 3, pool=True) == RING
+    assert conv_choice(4, 1, 64, 64, 12, 12, 3, pool=True) == HALO       # width not a power of two
+    assert conv_choice(4, 1, 64, 64, 14, 14, 3, stride=2) == HALO_LEAN
+    assert conv_choice(8, 1, 64, 64, 7, 7, 3, state=False) is None       # state between blocks
+    assert conv_choice(4, 1, 64, 70, 7, 7, 3, lif=(2.0, -1.0, 0.0, 1, 1)) == HALO
+    assert conv_choice(4, 1, 512, 64, 1, 1, 1) == RING
+    assert conv_choice(4, 512, 512, 4096, 1, 1, 1) == GENERAL            # several rounds, 1x1 map
