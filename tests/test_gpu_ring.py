@@ -10,11 +10,12 @@ import torch
 import oracle
 from catfuse_amd import runtime
 from catfuse_amd.runtime import EPI_LIF, EPI_POOL, ConvLIFRunner
+from choice import HALO, HALO_LEAN, RING, conv_choice
 from parity import lif_parity
 
 pytestmark = pytest.mark.gpu
 
-# T, B, Cin, Cout, H, W, k: all small enough for one round of workgroups
+# T, B, Cin, Cout, H, W, k: one round of workgroups but for the last two
 SHAPES = [
     (4, 1, 64, 64, 7, 7, 3), (3, 2, 32, 32, 5, 9, 3), (6, 3, 96, 64, 13, 11, 3),
     (4, 1, 40, 64, 14, 14, 3), (8, 1, 33, 64, 16, 15, 3), (4, 1, 64, 64, 30, 30, 3),
@@ -25,6 +26,7 @@ SHAPES = [
     (4, 30, 64, 704, 7, 7, 1),           # 64-channel tiles
     (4, 2, 64, 70, 7, 7, 3), (5, 1, 32, 5, 9, 9, 3), (4, 2, 64, 37, 8, 8, 1),
     (4, 30, 64, 690, 7, 7, 1),           # channels off 32 and off 64
+    (4, 600, 64, 1024, 1, 1, 3), (5, 300, 33, 288, 2, 3, 3),   # two rounds of workgroups
 ]
 POOLED = [(4, 1, 64, 64, 16, 16), (4, 3, 96, 64, 8, 8), (6, 5, 64, 64, 4, 4),
           (4, 33, 64, 96, 2, 2), (3, 2, 32, 32, 6, 4), (1, 4, 512, 512, 2, 2)]
@@ -70,6 +72,7 @@ def _tiled(r, x, v0, pool, ident):
 @pytest.mark.parametrize("ident,vin", [(False, False), (True, True)])
 def test_flat_tiles(cuda, shape, ident, vin):
     T, B, Ci, Co, H, W, k = shape
+    assert conv_choice(T, B, Ci, Co, H, W, k, ident=ident) == RING
     r, w, sc, sh = _layer(cuda, Ci, Co, k)
     g = torch.Generator().manual_seed(1)
     x = (torch.rand(T, B, Ci, H, W, generator=g) < 0.3).float()
@@ -96,6 +99,7 @@ def test_flat_tiles(cuda, shape, ident, vin):
 @pytest.mark.parametrize("vin", [False, True])
 def test_flat_tiles_pooled(cuda, shape, vin):
     T, B, Ci, Co, H, W = shape
+    assert conv_choice(T, B, Ci, Co, H, W, 3, pool=True) == RING
     r = _layer(cuda, Ci, Co, 3)[0]
     g = torch.Generator().manual_seed(2)
     xl = _lazy((torch.rand(T, B, Ci, H, W, generator=g) < 0.3).float(), cuda)
@@ -120,7 +124,8 @@ def test_flat_tiles_zero_input(cuda, k, pool):
 
 @pytest.mark.parametrize("Co", [1, 31, 40, 70, 170])
 @pytest.mark.parametrize("k,stride,H,W,T,B", [(3, 1, 40, 33, 4, 3), (3, 2, 45, 61, 6, 2),
-                                              (1, 2, 31, 30, 4, 2), (3, 1, 35, 64, 9, 1)])
+                                              (1, 2, 31, 30, 4, 2), (3, 1, 35, 64, 9, 1),
+                                              (3, 1, 40, 65, 4, 3)])
 @pytest.mark.parametrize("v_th", [0.3, -1.0])
 def test_channels_off_32(cuda, Co, k, stride, H, W, T, B, v_th):
     """The 8x8-tile kernel at channel counts off 32: the spikes, the sums with
@@ -136,6 +141,9 @@ def test_channels_off_32(cuda, Co, k, stride, H, W, T, B, v_th):
     Ho, Wo = r.out_hw(H, W)
     i0 = torch.randint(0, 3, (T, B, Co, Ho, Wo), generator=g).float()
     for ident in (None, i0):
+        if stride == 2 or W > 62:       # (else the flat-tile kernel may take it)
+            assert conv_choice(T, B, Ci, Co, H, W, k, stride=stride, ident=ident is not None,
+                               lif=(2.0, v_th, 0.0, 1, 1)) == (HALO_LEAN if v_th > 0 else HALO)
         for inp in (x, torch.zeros_like(x)):
             xl = _lazy(inp, cuda)
             y, v = r.run_mfma(xl, identity=None if ident is None else _lazy(ident, cuda))
