@@ -56,32 +56,34 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t attn_rsrc(const void* base, ui
 }
 
 // Every product and sum here is exact (integers), so the order of the sums is
-// free and four time steps run side by side: waves 2 t and 2 t + 1 take step t
-// of the block.  A step's K and V are staged transposed ([d][token], two
-// tokens a word, so each MFMA operand is one 16-byte read; rows of NM / 2 + 4
+// free and TB time steps run side by side, WPS waves on each: waves WPS t ..
+// take step t of the block.  A step's K and V are staged transposed ([d][token],
+// two tokens a word, so each MFMA operand is one 16-byte read; rows of NM / 2 + 4
 // words spread an operand's 32 rows over all banks).  Each wave sums K^T V
 // itself, and its accumulators are the second product's B operand as they
 // lie: the k slots of Y = Q (K^T V) are assigned to the rows d a lane holds,
 // and Q is read in that order.  The sums then meet in LDS (over the staged
 // tokens), and a thread runs the LIF over the block's steps for 8 channels of a
 // token and stores 16 bytes a step.  Bound by latency: one round of loads, one
-// transpose and two barriers a block of four steps, where one step after
-// another took that per step.  Measured (T = 4, 196 tokens, 12 heads): one
-// image 27 -> 14.5 us, 32 images (384 workgroups, one a CU) 39 -> 33.5.
-template <int NM, int LM>
-__global__ __launch_bounds__(512) void spike_attention_kernel(AttnArgs a) {
-  constexpr int TB = 4, KW = NM / 2 + 4, ZLD = DH + 4;
+// transpose and two barriers a block.  Four steps a block (TB 4, WPS 2) take
+// that once for T = 4: one image (196 tokens, 12 heads) 11.3 us, where a
+// workgroup of four waves that took one step after another took 22.6.
+// (launch_attention says where one step a block is the faster one.)
+template <int NM, int TB, int WPS, int LM>
+__global__ __launch_bounds__(64 * TB * WPS) void spike_attention_kernel(AttnArgs a) {
+  constexpr int NT = 64 * TB * WPS, KW = NM / 2 + 4, ZLD = DH + 4;
   constexpr int KV_BYTES = 2 * TB * DH * KW * 4, Z_BYTES = TB * NM * ZLD * 4;
-  constexpr int SU = NM / 64;               // staged units of a thread (2 tokens x 8 channels)
-  constexpr int MAXT = NM / 64;             // 32-token tiles of Y per wave at most
-  constexpr int LU = (NM + 127) / 128;      // LIF units of a thread (a token x 8 channels)
+  // staged units of a thread (2 tokens x 8 channels; units past NM are not staged)
+  constexpr int SU = (2 * NM + 64 * WPS - 1) / (64 * WPS);
+  constexpr int MAXT = (NM / 32 + WPS - 1) / WPS;   // 32-token tiles of Y per wave at most
+  constexpr int LU = (4 * NM + NT - 1) / NT;        // LIF units of a thread (a token x 8 channels)
   __shared__ __attribute__((aligned(16))) char smem[KV_BYTES > Z_BYTES ? KV_BYTES : Z_BYTES];
-  __shared__ unsigned any_sh[8];
+  __shared__ unsigned any_sh[TB * WPS];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int hi = lane >> 5, col = lane & 31;
-  const int ts = wave >> 1, wh = wave & 1;  // this wave's step of the block, its half of the tiles
+  const int ts = wave / WPS, wh = wave % WPS;  // this wave's step of the block, its first tile
   const int N = a.N, C = a.heads * DH;
   const int nks = (N + 15) / 16;            // 16-token MFMA steps of K^T V
   const int ntile = (N + 31) / 32;          // 32-token row tiles of Y
@@ -111,13 +113,13 @@ __global__ __launch_bounds__(512) void spike_attention_kernel(AttnArgs a) {
   const int work = xcd * (nwork >> 3) + min(xcd, nwork & 7) + ((int)blockIdx.x >> 3);
   const int b = work / a.heads, h = work % a.heads;
 
-  // membrane potentials: unit i is token tid / 4 + 128 i, channels 8 (tid % 4) ..
+  // membrane potentials: unit i is token tid / 4 + NT / 4 i, channels 8 (tid % 4) ..
   const int ln = tid >> 2, lc = (tid & 3) * 8;
   float v[LU][8];
   const float v0 = lif_initial_v(a.lif);
 #pragma unroll
   for (int i = 0; i < LU; ++i) {
-    const int n = ln + 128 * i;
+    const int n = ln + NT / 4 * i;
     const float* vs = a.v_in + ((size_t)b * N + n) * C + h * DH + lc;
 #pragma unroll
     for (int j = 0; j < 8; ++j) v[i][j] = a.v_in != nullptr && n < N ? vs[j] : v0;
@@ -142,11 +144,11 @@ __global__ __launch_bounds__(512) void spike_attention_kernel(AttnArgs a) {
       // every load of the block is issued before its first use (rows beyond
       // N read zeros, out of the buffers' range)
       auto off = [&](int n, int c) { return n < N ? (uint32_t)((n * a.pitch + c) * 2) : 0x80000000u; };
-      const int g = tid & 127;
+      const int g = tid & (64 * WPS - 1);
       u32x4 kx[SU][2], vx[SU][2];
 #pragma unroll
       for (int i = 0; i < SU; ++i) {
-        const int u = g + 128 * i, n = (u >> 2) * 2, c = (u & 3) * 8;
+        const int u = g + 64 * WPS * i, n = (u >> 2) * 2, c = (u & 3) * 8;
 #pragma unroll
         for (int e = 0; e < 2; ++e) {
           kx[i][e] = __builtin_amdgcn_raw_buffer_load_b128(rk, off(n + e, c), 0, 0);
@@ -163,10 +165,10 @@ __global__ __launch_bounds__(512) void spike_attention_kernel(AttnArgs a) {
 #pragma unroll
           for (int e = 0; e < 2; ++e)
             qx[i][s][e] = __builtin_amdgcn_raw_buffer_load_b64(
-                rq, off((wh + 2 * i) * 32 + col, 16 * s + 8 * e + 4 * hi), 0, 0);
+                rq, off((wh + WPS * i) * 32 + col, 16 * s + 8 * e + 4 * hi), 0, 0);
 #pragma unroll
       for (int i = 0; i < SU; ++i) {
-        const int u = g + 128 * i, pr = u >> 2, c = (u & 3) * 8;
+        const int u = g + 64 * WPS * i, pr = u >> 2, c = (u & 3) * 8;
         if (2 * pr < 16 * nks) {
 #pragma unroll
           for (int j = 0; j < 8; ++j) {
@@ -200,7 +202,7 @@ __global__ __launch_bounds__(512) void spike_attention_kernel(AttnArgs a) {
     }
 #pragma unroll
     for (int i = 0; i < MAXT; ++i) {
-      const int tile = wh + 2 * i;
+      const int tile = wh + WPS * i;
       if (tile >= ntile) break;
 #pragma unroll
       for (int r = 0; r < 16; ++r)
@@ -209,7 +211,7 @@ __global__ __launch_bounds__(512) void spike_attention_kernel(AttnArgs a) {
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < LU; ++i) {
-      const int n = ln + 128 * i;
+      const int n = ln + NT / 4 * i;
       if (n >= N) break;
 #pragma unroll
       for (int t = 0; t < TB; ++t) {
@@ -239,7 +241,7 @@ __global__ __launch_bounds__(512) void spike_attention_kernel(AttnArgs a) {
   if (a.v_out) {
 #pragma unroll
     for (int i = 0; i < LU; ++i) {
-      const int n = ln + 128 * i;
+      const int n = ln + NT / 4 * i;
       if (n >= N) break;
       float* vd = a.v_out + ((size_t)b * N + n) * C + h * DH + lc;
 #pragma unroll
@@ -253,19 +255,32 @@ __global__ __launch_bounds__(512) void spike_attention_kernel(AttnArgs a) {
     if (tid == 0) {
       unsigned w = 0u;
 #pragma unroll
-      for (int i = 0; i < 8; ++i) w |= any_sh[i];
+      for (int i = 0; i < TB * WPS; ++i) w |= any_sh[i];
       cf_count_publish(a.nz_out, w ? 1ull : 0ull, blockIdx.x, gridDim.x);
     }
   }
 }
 
-// (Workgroups of fewer tokens need less LDS, so more share a CU.)
+// Workgroups of fewer tokens need less LDS, so more share a CU.  Four steps of
+// more than 128 tokens take 147 KB, one workgroup a CU: launches of more
+// workgroups than CUs then run in rounds, and steps that do not exist (T off 4)
+// cost as much as those that do.  They take one step a block, eight waves on it
+// (37 KB, four workgroups a CU).  Measured (us, four steps / one step a block),
+// 196 tokens: 384 workgroups, T = 1 20.2 / 8.8, 4 26.5 / 21.7, 5 42.3 / 25.1; 1536,
+// T = 1 58.1 / 20.9, 2 67.5 / 31.5; 256 tokens, 768, T = 4 49.3 / 37.7; but 256
+// workgroups, 196 tokens, T = 4 16.6 / 18.8.  Up to 128 tokens four steps are
+// the faster choice at one image and both lie far below what one step after
+// another took.
 template <int LM>
 void launch_attention(const AttnArgs& a, hipStream_t st) {
   const dim3 grid((unsigned)(a.B * a.heads)), block(512);
-  if (a.N <= 64) hipLaunchKernelGGL((spike_attention_kernel<64, LM>), grid, block, 0, st, a);
-  else if (a.N <= 128) hipLaunchKernelGGL((spike_attention_kernel<128, LM>), grid, block, 0, st, a);
-  else hipLaunchKernelGGL((spike_attention_kernel<NMAX, LM>), grid, block, 0, st, a);
+  const int cus = cf_cu_count() > 0 ? cf_cu_count() : 256;
+  if (a.N <= 64) hipLaunchKernelGGL((spike_attention_kernel<64, 4, 2, LM>), grid, block, 0, st, a);
+  else if (a.N <= 128)
+    hipLaunchKernelGGL((spike_attention_kernel<128, 4, 2, LM>), grid, block, 0, st, a);
+  else if (grid.x <= (unsigned)cus)
+    hipLaunchKernelGGL((spike_attention_kernel<NMAX, 4, 2, LM>), grid, block, 0, st, a);
+  else hipLaunchKernelGGL((spike_attention_kernel<NMAX, 1, 8, LM>), grid, block, 0, st, a);
 }
 
 // ---------------------------------------------------------------------------

@@ -131,6 +131,20 @@ __host__ __device__ inline bool cf_lif_silent_at_rest(const LifParams& p) {
   return (p.hard ? p.v_reset : 0.0f) < p.v_th;
 }
 
+// Compute units of the current device (cached per device), or 0 when the
+// runtime does not say.
+static inline int cf_cu_count() {
+  static int cache[64] = {0};
+  int dev = 0;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+  if (cache[dev] == 0) {
+    int n = 0;
+    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) n = 0;
+    cache[dev] = n > 0 ? n : -1;
+  }
+  return cache[dev] > 0 ? cache[dev] : 0;
+}
+
 // The kernels a fused conv launch may take (CF_CONV_* of cf_conv_mfma_choice).
 enum { CONV_BY_GENERAL = 0, CONV_BY_HALO = 1, CONV_BY_HALO_LEAN = 2, CONV_BY_RING = 3 };
 

@@ -88,18 +88,4 @@ __device__ __forceinline__ unsigned lds_addr(const void* p) {
 enum { EPI_LIF = 0, EPI_Z = 1, EPI_POOL = 2 };
 enum { ID_ADD_SPIKE = 1, ID_ADD_Z = 2 };
 
-// Compute units of the current device (cached per device), or 0 when the
-// runtime does not say.
-inline int cf_cu_count() {
-  static int cache[64] = {0};
-  int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
-  if (cache[dev] == 0) {
-    int n = 0;
-    if (hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) n = 0;
-    cache[dev] = n > 0 ? n : -1;
-  }
-  return cache[dev] > 0 ? cache[dev] : 0;
-}
-
 }  // namespace

@@ -14,6 +14,17 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("N", [1, 15, 17, 33, 63, 64, 65, 127, 128, 129, 200, 255, 256])
 @pytest.mark.parametrize("T,B,heads,cp_pad", [(1, 1, 1, 0), (5, 2, 3, 0), (4, 9, 1, 4)])
 def test_attention_edges(cuda, N, T, B, heads, cp_pad):
+    _check_attention(cuda, N, T, B, heads, cp_pad)
+
+
+@pytest.mark.parametrize("N", [128, 129, 196, 255, 256])
+@pytest.mark.parametrize("T,B,heads,cp_pad", [(1, 257, 1, 0), (2, 65, 4, 0), (5, 33, 8, 4)])
+def test_attention_more_workgroups_than_cus(cuda, N, T, B, heads, cp_pad):
+    """One step a block (more than 128 tokens, more workgroups than CUs)."""
+    _check_attention(cuda, N, T, B, heads, cp_pad)
+
+
+def _check_attention(cuda, N, T, B, heads, cp_pad):
     from catfuse_amd import runtime, snn
     C = 32 * heads
     g = torch.Generator().manual_seed(N + T)
