@@ -685,6 +685,19 @@ bool cf_conv_ring(int* rc, const void* x, const void* w_packed, const float* alp
     // 14 / 15; 1,568 rows 1536 -> 384 36 (300 workgroups) / 26 / 39; 784 rows
     // 384 -> 1152 22 (468) / 16 / 20, 384 -> 1536 30 (624) / 28 (312) / 21.
     if (n32 > cus && n64 > cus) return false;
+    // Few chunks do not pay for filling the rings.  Up to four steps (more take
+    // conv_halo.hip two blocks), here / there: 32 -> 32 channels, 784 rows, T = 1
+    // 6.4 / 5.6, 2 6.6 / 6.2, 3 1.01 of it, 4 0.96; 64 -> 64 T = 1 6.6 / 6.1, 2 1.02
+    // of it, 3 0.97; 96 1.01, 0.96.  64-channel tiles where conv_halo.hip has its
+    // one round too: 1,568 rows, 96 -> 512 T = 1 8.7 / 7.3, 192 1.05 of it, 224 1.02,
+    // 256 0.99, T = 4 1.10, 1.00, 0.98, 0.94; where it has two (1,470 rows -> 704, 7x7
+    // maps) as 32-channel ones: 96 channels T = 1 1.02, 2 0.98.  (Maps below 4x4
+    // take the general kernel instead, two to ten times as long.)
+    if (T <= 4 && H >= 4 && W >= 4) {
+      const int64_t nch = Cp / KC;
+      const int64_t halo_wg = B * ((H + 7) / 8) * ((W + 7) / 8) * (Coutp / 64);
+      if (nch + T < 5 || (n32 > cus && halo_wg <= cus && nch < 7)) return false;
+    }
     mw = n32 <= cus ? 1 : 2;
   }
   a.ncb = mw == 2 ? (int)(Coutp / 64) : (int)((Cout + 31) / 32);

@@ -318,4 +318,17 @@ def test_flat_tile_kernel_bounds():
     assert conv_choice(8, 1, 64, 64, 7, 7, 3, state=False) is None       # state between blocks
     assert conv_choice(4, 1, 64, 70, 7, 7, 3, lif=(2.0, -1.0, 0.0, 1, 1)) == HALO
     assert conv_choice(4, 1, 512, 64, 1, 1, 1) == RING
+    # 1x1 with few input channels: only from some steps on, where the 8x8 tiles
+    # are the other choice
+    for Ci, T0 in ((32, 4), (64, 3), (96, 2), (128, 1)):
+        for T in range(1, 9):
+            assert conv_choice(T, 1, Ci, 64, 8, 8, 1) == (RING if T >= T0 else HALO_LEAN)
+            assert conv_choice(T, 4, Ci, 64, 3, 3, 1) == RING
+    # 64-channel tiles in one round, beside one round or two of 8x8 tiles
+    for Ci in range(32, 320, 32):
+        for T in (1, 4, 5):
+            assert (conv_choice(T, 8, Ci, 512, 14, 14, 1)
+                    == (RING if T > 4 or Ci >= 224 else HALO_LEAN)), (Ci, T)
+            assert (conv_choice(T, 30, Ci, 704, 7, 7, 1)
+                    == (RING if Ci // 32 + T >= 5 else HALO_LEAN)), (Ci, T)
     assert conv_choice(4, 512, 512, 4096, 1, 1, 1) == GENERAL            # several rounds, 1x1 map
