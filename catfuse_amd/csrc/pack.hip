@@ -210,17 +210,50 @@ __global__ __launch_bounds__(256) void scan_nhwc_kernel(
 
 // fp16 NHWC [NB][HW][cp] -> fp32 NCHW [NB][C][HW]: materialises the fp32
 // view of a fused conv output that was kept only as its NHWC copy, read where
-// its producer left it (desc, nullable: an all-zero copy gives zeros).  A
-// block moves 64 pixels x 64 channels through LDS, the reverse of
-// pack_kernel: a channel pair's halves are one word of a pixel's 33-word row;
-// reads are 128-byte runs per pixel, writes 16 bytes (four pixels of a channel)
-// a lane (128 images of 256 x 14 x 14 11.7 us, of 128 x 28 x 28 18.2; 4-byte
-// stores of 32-channel tiles took 12.5 and 17.6).  What reading through the
-// descriptor saves is the launch that filled unwritten copies first, 4.5 us of
-// the GPU's time and 5 of the host's.
+// its producer left it (desc, nullable: an all-zero copy gives zeros).  What
+// reading through the descriptor saves is the launch that filled unwritten
+// copies first, 4.5 us of the GPU's time and 5 of the host's.
 // XT: the copy's element, fp16 or one byte per channel (uint8_t).
+//
+// A block moves 64 pixels x 32 channels through LDS (reads: 64-byte runs per
+// pixel; writes: 256-byte runs per channel, a wave's 4-byte stores side by
+// side), or the wide form below (nhwc_to_nchw says where).
 template <typename XT>
 __global__ __launch_bounds__(256) void nhwc_to_nchw_kernel(
+    const XT* __restrict__ xp_own, const CfOutDesc* __restrict__ desc, float* __restrict__ out,
+    int64_t C, int64_t HW, int64_t cp) {
+  typedef XT x8 __attribute__((ext_vector_type(8)));
+  __shared__ float tile[CC][PX + 1];
+  const int tid = threadIdx.x;
+  const XT* const xp = cf_copy_source(desc, xp_own);
+  const int64_t n = blockIdx.z;
+  const int64_t hw0 = (int64_t)blockIdx.x * PX;
+  const int64_t c0 = (int64_t)blockIdx.y * CC;
+  {
+    // read: 4 threads per pixel, 8 channels (16 or 8 bytes) each
+    const int px = tid / 4, part = tid % 4;
+    x8 v = {};
+    if (xp != nullptr && hw0 + px < HW && c0 + part * 8 < cp)
+      v = *reinterpret_cast<const x8*>(xp + ((n * HW + hw0 + px) * cp + c0 + part * 8));
+#pragma unroll
+    for (int j = 0; j < 8; ++j) tile[part * 8 + j][px] = (float)v[j];
+  }
+  __syncthreads();
+  // write: 64 consecutive pixels of one channel per 64 threads
+  const int px = tid % PX;
+#pragma unroll
+  for (int i = 0; i < CC / 4; ++i) {
+    const int cl = tid / PX + 4 * i;
+    const int64_t c = c0 + cl;
+    if (c < C && hw0 + px < HW) out[(n * C + c) * HW + hw0 + px] = tile[cl][px];
+  }
+}
+
+// The wide form: 64 pixels x 64 channels, the reverse of pack_kernel: a channel
+// pair's halves are one word of a pixel's 33-word row; reads are 128-byte runs
+// per pixel, writes 16 bytes (four pixels of a channel) a lane.
+template <typename XT>
+__global__ __launch_bounds__(256) void nhwc_to_nchw_wide_kernel(
     const XT* __restrict__ xp_own, const CfOutDesc* __restrict__ desc, float* __restrict__ out,
     int64_t C, int64_t HW, int64_t cp) {
   typedef XT x8 __attribute__((ext_vector_type(8)));
@@ -676,9 +709,29 @@ static int nhwc_to_nchw(const void* xp, const void* desc, float* out, int64_t NB
     return (int)hipErrorInvalidValue;
   if (NB == 0) return 0;
   const int64_t HW = H * W;
-  dim3 grid(cf_blocks(HW, PX), (unsigned)((C + 63) / 64), (unsigned)NB);
-  hipLaunchKernelGGL(nhwc_to_nchw_kernel<XT>, grid, dim3(256), 0, (hipStream_t)stream,
-                     (const XT*)xp, (const CfOutDesc*)desc, out, C, HW, cp);
+  // The wide form where its tiles waste no half (an even number of 32-channel
+  // groups) and either maps are so small that a tile is mostly channels, or an
+  // fp16 copy is so large that HBM is what bounds it; rows of about 4 KB and its
+  // multiples put its 16 channels' stores on the same channels of the memory.
+  // Measured (us, 32 channels / wide): 488 x 512 channels of 2 x 2 8.3 / 6.4, 3906 x
+  // 256 of 1 x 1 25 / 14.4; 298 x 512 of 14 x 14 47.5 / 40, 149 x 64 of 56 x 56 35.5 /
+  // 30.3, but 59 x 512 of 14 x 14 11 / 11, 71 x 90 of 32 x 32 7.7 / 11.2, 742 x 40 of
+  // 30 x 34 37.2 / 39.8, 128 x 512 of 7 x 7 5.5 / 6.5, 49 x 332 of 10 x 10 4.5 / 5.2,
+  // bytes of 128 x 256 of 14 x 14 9.9 / 11.3.
+  const int64_t tiles = (HW + PX - 1) / PX * ((C + 63) / 64) * NB;
+  const bool wide = (C + CC - 1) / CC % 2 == 0 &&
+                    (HW <= 16 ? tiles >= 900
+                              : sizeof(XT) == 2 && HW >= 100 && (HW + 32) % 1024 > 64 && tiles >= 3000);
+  if (wide)
+    hipLaunchKernelGGL(nhwc_to_nchw_wide_kernel<XT>,
+                       dim3(cf_blocks(HW, PX), (unsigned)((C + 63) / 64), (unsigned)NB), dim3(256),
+                       0, (hipStream_t)stream, (const XT*)xp, (const CfOutDesc*)desc, out, C, HW,
+                       cp);
+  else
+    hipLaunchKernelGGL(nhwc_to_nchw_kernel<XT>,
+                       dim3(cf_blocks(HW, PX), (unsigned)((C + CC - 1) / CC), (unsigned)NB),
+                       dim3(256), 0, (hipStream_t)stream, (const XT*)xp, (const CfOutDesc*)desc, out,
+                       C, HW, cp);
   return (int)hipGetLastError();
 }
 

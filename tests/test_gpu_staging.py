@@ -97,3 +97,43 @@ def test_maxpool_order_with_nan(cuda, H, W, k, s, p):
                 m = torch.where(q > m, q, m)
             want[..., oh, ow] = m
     assert torch.equal(y.cpu().nan_to_num(7.0), want.nan_to_num(7.0))
+
+
+def _copies(NB, H, W, C, cp, dtype, cuda):
+    g = torch.Generator(device=cuda).manual_seed(C)
+    c = torch.randint(0, 4, (2, NB, H, W, cp), device=cuda, generator=g).to(dtype)
+    c[..., C:] = 0
+    return c[0].contiguous(), c[1].contiguous()
+
+
+def _descs(alias, cuda):
+    """Absent, written, all zero, an alias (the 16 bytes of a CfOutDesc)."""
+    return [None] + [torch.tensor([k, alias.data_ptr() if k == 2 else 0], dtype=torch.int64,
+                                  device=cuda) for k in (0, 1, 2)]
+
+
+# both forms of the fp32 pass, tiles partly filled in pixels and channels (the last
+# six: 64-channel tiles)
+@pytest.mark.parametrize("NB,C,H,W", [
+    (1, 1, 1, 1), (3, 33, 5, 13), (2, 64, 8, 8), (3, 65, 7, 9), (2, 96, 9, 29), (1, 130, 3, 43),
+    (2, 70, 32, 32), (450, 100, 3, 3), (900, 33, 1, 1), (901, 64, 4, 4), (1500, 40, 1, 101),
+    (47, 64, 17, 251), (4, 1000, 61, 64)])
+def test_materialise_edges(cuda, NB, C, H, W):
+    """The fp32 form of an fp16 copy read through every kind of descriptor, and
+    of a byte copy."""
+    lib, p, st = runtime._hip.lib(), runtime.ptr, runtime._hip.stream(cuda)
+    cp = runtime.pad32(C) + (8 if C % 2 else 0)
+    copy, other = _copies(NB, H, W, C, cp, torch.float16, cuda)
+    out = torch.empty(NB, C, H, W, device=cuda)
+    want = copy[..., :C].permute(0, 3, 1, 2).float()
+    wants = (want, want, torch.zeros_like(want), other[..., :C].permute(0, 3, 1, 2).float())
+    for d, w in zip(_descs(other, cuda), wants):
+        out.fill_(-1.0)
+        assert lib.cf_copy_to_f32(p(copy), p(d), p(out), NB, C, H, W, cp, 0, st) == 0
+        assert torch.equal(out, w)
+    out.fill_(-1.0)
+    assert lib.cf_nhwc_to_nchw(p(copy), p(out), NB, C, H, W, cp, st) == 0
+    assert torch.equal(out, want)
+    out.fill_(-1.0)
+    assert lib.cf_nhwc_to_nchw_u8(p(copy.to(torch.uint8)), p(out), NB, C, H, W, cp, st) == 0
+    assert torch.equal(out, want)
