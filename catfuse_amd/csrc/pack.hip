@@ -353,9 +353,12 @@ __global__ __launch_bounds__(256) void global_avgpool_nhwc_kernel(
 // -> its fp16 copy [NB][P][cp] (channels C..cp-1 zero), the nonzero count
 // (published in a count block) and the exactness status: the staging of a
 // fused linear's input, which the matrix-core kernels read as an NHWC image
-// of P pixels.  Bound by HBM: a thread takes two 8-channel chunks a pass
-// (grid-stride), their 16-byte loads in flight together (25,088 rows of 384:
-// 21 -> 11 us against one chunk a pass in 4-byte loads).
+// of P pixels.  A thread takes U 8-channel chunks a pass (grid-stride).  Bound by
+// HBM when large: two chunks, their 16-byte loads in flight together (25,088 rows
+// of 384: 22 -> 11.9 us against one chunk in 4-byte loads).  Bound by a launch's
+// latency when small: one chunk, whose eight predicated loads are one round
+// (681 rows of 5: 4.4 us with two chunks of two load widths, 3.5 so).
+template <int U>
 __global__ __launch_bounds__(256) void pack_tokens_kernel(
     const float* __restrict__ x, int64_t rows, int C, int cp, _Float16* __restrict__ xp,
     unsigned long long* __restrict__ nnz, uint32_t* __restrict__ status) {
@@ -363,48 +366,67 @@ __global__ __launch_bounds__(256) void pack_tokens_kernel(
   __shared__ unsigned int inexact_sh;
   if (threadIdx.x == 0) { cnt_sh = 0; inexact_sh = 0; }
   __syncthreads();
-  const uint32_t nc8 = (uint32_t)cp / 8u;
   unsigned int cnt = 0;
   bool inexact = false;
-  const int64_t units = rows * nc8, step = (int64_t)gridDim.x * 256;
-  // (32-bit unit decode wherever it fits: a 64-bit division by a run-time
-  // value costs more than the unit's own work)
-  const bool small = units + 2 * step < ((int64_t)1 << 32);
-  // Two units a pass, their four 16-byte loads in flight together.
-  for (int64_t u0 = (int64_t)blockIdx.x * 256 + threadIdx.x; u0 < units; u0 += 2 * step) {
-    float v[2][8];
-    int64_t dst[2];
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      const int64_t u = u0 + k * step;
-      const bool live = u < units;
-      const int64_t r = small ? (int64_t)((uint32_t)u / nc8) : u / nc8;
-      const int c0 = (int)(u - r * nc8) * 8;
-      dst[k] = live ? r * cp + c0 : -1;
-      const float* src = x + r * C + c0;
-      if (live && c0 + 8 <= C) {
-        const f32x4u q0 = *reinterpret_cast<const f32x4u*>(src);
-        const f32x4u q1 = *reinterpret_cast<const f32x4u*>(src + 4);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) { v[k][j] = q0.v[j]; v[k][4 + j] = q1.v[j]; }
-      } else {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) v[k][j] = (live && c0 + j < C) ? src[j] : 0.0f;
-      }
-    }
-#pragma unroll
-    for (int k = 0; k < 2; ++k) {
-      if (dst[k] < 0) continue;
+  if constexpr (U == 1) {
+    const int nc8 = cp / 8;
+    for (int64_t u = (int64_t)blockIdx.x * 256 + threadIdx.x; u < rows * nc8;
+         u += (int64_t)gridDim.x * 256) {
+      const int64_t r = u / nc8;
+      const int c0 = (int)(u % nc8) * 8;
       _Float16 o[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        const float f = v[k][j];
-        const _Float16 hv = (_Float16)f;
-        inexact |= ((float)hv != f);
-        cnt += (f != 0.0f) ? 1u : 0u;
+        const float v = (c0 + j < C) ? x[r * C + c0 + j] : 0.0f;
+        const _Float16 hv = (_Float16)v;
+        inexact |= ((float)hv != v);
+        cnt += (v != 0.0f) ? 1u : 0u;
         o[j] = hv;
       }
-      *reinterpret_cast<uint4*>(xp + dst[k]) = *reinterpret_cast<const uint4*>(o);
+      *reinterpret_cast<uint4*>(xp + r * cp + c0) = *reinterpret_cast<const uint4*>(o);
+    }
+  } else {
+    const uint32_t nc8 = (uint32_t)cp / 8u;
+    const int64_t units = rows * nc8, step = (int64_t)gridDim.x * 256;
+    // (32-bit unit decode wherever it fits: a 64-bit division by a run-time
+    // value costs more than the unit's own work)
+    const bool small = units + U * step < ((int64_t)1 << 32);
+    for (int64_t u0 = (int64_t)blockIdx.x * 256 + threadIdx.x; u0 < units; u0 += U * step) {
+      float v[U][8];
+      int64_t dst[U];
+#pragma unroll
+      for (int k = 0; k < U; ++k) {
+        const int64_t u = u0 + k * step;
+        dst[k] = -1;
+        if (k > 0 && u >= units) continue;
+        const int64_t r = small ? (int64_t)((uint32_t)u / nc8) : u / nc8;
+        const int c0 = (int)(u - r * nc8) * 8;
+        dst[k] = r * cp + c0;
+        const float* src = x + r * C + c0;
+        if (c0 + 8 <= C) {
+          const f32x4u q0 = *reinterpret_cast<const f32x4u*>(src);
+          const f32x4u q1 = *reinterpret_cast<const f32x4u*>(src + 4);
+#pragma unroll
+          for (int j = 0; j < 4; ++j) { v[k][j] = q0.v[j]; v[k][4 + j] = q1.v[j]; }
+        } else {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) v[k][j] = c0 + j < C ? src[j] : 0.0f;
+        }
+      }
+#pragma unroll
+      for (int k = 0; k < U; ++k) {
+        if (dst[k] < 0) continue;
+        _Float16 o[8];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          const float f = v[k][j];
+          const _Float16 hv = (_Float16)f;
+          inexact |= ((float)hv != f);
+          cnt += (f != 0.0f) ? 1u : 0u;
+          o[j] = hv;
+        }
+        *reinterpret_cast<uint4*>(xp + dst[k]) = *reinterpret_cast<const uint4*>(o);
+      }
     }
   }
   if (nnz) {
@@ -420,10 +442,26 @@ __global__ __launch_bounds__(256) void pack_tokens_kernel(
 }
 
 // fp16 [NB][P][cp] -> fp32 [NB][P][C]: the fp32 form of a token-major fused
-// output kept only as its fp16 copy.  A thread takes an 8-channel chunk of a row (one 16-byte
-// load, two 16-byte stores): 25,088 rows of 384 20.6 -> 14.4 us against an
-// element a thread.
+// output kept only as its fp16 copy.  An element a thread, side by side, or a
+// thread takes an 8-channel chunk of a row (one 16-byte load, two 16-byte stores):
+// tokens_to_f32 says where.
 __global__ __launch_bounds__(256) void tokens_to_f32_kernel(
+    const _Float16* __restrict__ xp_own, const CfOutDesc* __restrict__ desc,
+    float* __restrict__ out, int64_t rows, int C, int cp) {
+  const _Float16* const xp = cf_copy_source(desc, xp_own);   // nullptr: all zero
+  const int64_t e0 = (int64_t)blockIdx.x * 256 + threadIdx.x, step = (int64_t)gridDim.x * 256;
+  if (xp == nullptr) {
+    for (int64_t e = e0; e < rows * C; e += step) out[e] = 0.0f;
+    return;
+  }
+  for (int64_t e = e0; e < rows * C; e += step) {
+    const int64_t r = e / C;
+    const int c = (int)(e % C);
+    out[e] = (float)xp[r * cp + c];
+  }
+}
+
+__global__ __launch_bounds__(256) void tokens_to_f32_chunks_kernel(
     const _Float16* __restrict__ xp_own, const CfOutDesc* __restrict__ desc,
     float* __restrict__ out, int64_t rows, int C, int cp) {
   const _Float16* const xp = cf_copy_source(desc, xp_own);   // nullptr: all zero
@@ -740,10 +778,20 @@ static int tokens_to_f32(const void* xp, const void* desc, float* out, int64_t r
   if (!xp || !out || rows < 0 || C <= 0 || cp < C || rows * cp > ((int64_t)1 << 40))
     return (int)hipErrorInvalidValue;
   if (rows == 0) return 0;
-  const int64_t n = rows * ((C + 7) / 8);
-  const unsigned grid = (unsigned)((n + 255) / 256 < 16384 ? (n + 255) / 256 : 16384);
-  hipLaunchKernelGGL(tokens_to_f32_kernel, dim3(grid), dim3(256), 0, (hipStream_t)stream,
-                     (const _Float16*)xp, (const CfOutDesc*)desc, out, rows, (int)C, (int)cp);
+  // Chunks where HBM bounds the pass: 50,176 rows of 384 26 -> 22 us; 3,136 of 384
+  // equal; rows that chunks do not fill cost a second, element-wise round: 784 rows
+  // of 100 2.6 -> 3.1, 100,000 of 33 6.5 -> 7.2, 50,176 of 257 19.3 -> 17.4.
+  const int64_t n = rows * C;
+  const bool chunks = C % 8 == 0 ? n >= (1 << 21) : C >= 256 && n >= (1 << 23);
+  const int64_t units = chunks ? rows * ((C + 7) / 8) : n;
+  const int64_t wg = (units + 255) / 256, most = chunks ? 16384 : 4096;
+  const dim3 grid((unsigned)(wg < most ? wg : most));
+  if (chunks)
+    hipLaunchKernelGGL(tokens_to_f32_chunks_kernel, grid, dim3(256), 0, (hipStream_t)stream,
+                       (const _Float16*)xp, (const CfOutDesc*)desc, out, rows, (int)C, (int)cp);
+  else
+    hipLaunchKernelGGL(tokens_to_f32_kernel, grid, dim3(256), 0, (hipStream_t)stream,
+                       (const _Float16*)xp, (const CfOutDesc*)desc, out, rows, (int)C, (int)cp);
   return (int)hipGetLastError();
 }
 
@@ -826,11 +874,21 @@ CF_API int cf_pack_tokens(const float* x, int64_t rows, int64_t C, int64_t cp, v
     return (int)hipErrorInvalidValue;
   if (rows == 0) return 0;
   const int64_t units = rows * (cp / 8);
-  // (4,096 workgroups hold the card's loads in flight; more only add
-  // count-block atomics)
-  const unsigned grid = (unsigned)((units + 511) / 512 < 4096 ? (units + 511) / 512 : 4096);
-  hipLaunchKernelGGL(pack_tokens_kernel, dim3(grid), dim3(256), 0, (hipStream_t)stream, x, rows,
-                     (int)C, (int)cp, (_Float16*)xp, nnz, status);
+  // Two chunks a thread once a launch has enough of them for its loads to bound it:
+  // 3,136 rows of 256 (100,352 chunks) 5.4 -> 4.4 us, 784 of 384 (37,632) equal; later
+  // where chunks are padding or partial: 12,544 rows of 48 (100,352) 4.4 -> 4.9, of 100
+  // (200,704) 6.5 -> 5.3.  (4,096 workgroups hold the card's loads in flight; more
+  // only add count-block atomics.)
+  if (C >= 32 && units >= (8 * C >= 7 * cp ? 65536 : 196608))
+    hipLaunchKernelGGL(pack_tokens_kernel<2>,
+                       dim3((unsigned)((units + 511) / 512 < 4096 ? (units + 511) / 512 : 4096)),
+                       dim3(256), 0, (hipStream_t)stream, x, rows, (int)C, (int)cp, (_Float16*)xp,
+                       nnz, status);
+  else
+    hipLaunchKernelGGL(pack_tokens_kernel<1>,
+                       dim3((unsigned)((units + 255) / 256 < 2048 ? (units + 255) / 256 : 2048)),
+                       dim3(256), 0, (hipStream_t)stream, x, rows, (int)C, (int)cp, (_Float16*)xp,
+                       nnz, status);
   return (int)hipGetLastError();
 }
 

@@ -47,7 +47,11 @@ def test_pack_input_edges(cuda, shape, act):
     assert int(st) == 0
 
 
-@pytest.mark.parametrize("rows,C", [(1, 1), (7, 31), (513, 64), (130, 100), (1030, 384)])
+# (16,385 rows of 31 on: both sides of where two chunks a thread begin, and
+# 8-channel chunks of fp32 rows)
+@pytest.mark.parametrize("rows,C", [(1, 1), (7, 31), (513, 64), (130, 100), (1030, 384),
+                                    (16385, 31), (16384, 32), (16385, 100), (5500, 400),
+                                    (32770, 257), (32769, 64)])
 def test_pack_tokens_and_back(cuda, rows, C):
     x = _spikes((1, 1, rows, C), cuda, 1)
     cp = runtime.pad32(C)
@@ -136,4 +140,23 @@ def test_materialise_edges(cuda, NB, C, H, W):
     assert torch.equal(out, want)
     out.fill_(-1.0)
     assert lib.cf_nhwc_to_nchw_u8(p(copy.to(torch.uint8)), p(out), NB, C, H, W, cp, st) == 0
+    assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("rows,C,pad", [(1, 1, 0), (33, 40, 0), (130, 100, 4), (5500, 400, 0),
+                                        (32770, 257, 8), (32769, 64, 3)])
+def test_materialise_tokens_edges(cuda, rows, C, pad):
+    """The fp32 rows of a token-major copy read through every kind of descriptor."""
+    lib, p, st = runtime._hip.lib(), runtime.ptr, runtime._hip.stream(cuda)
+    cp = runtime.pad32(C) + pad
+    copy, other = (t.view(rows, cp) for t in _copies(1, 1, rows, C, cp, torch.float16, cuda))
+    out = torch.empty(rows, C, device=cuda)
+    want = copy[:, :C].float()
+    wants = (want, want, torch.zeros_like(want), other[:, :C].float())
+    for d, w in zip(_descs(other, cuda), wants):
+        out.fill_(-1.0)
+        assert lib.cf_copy_to_f32(p(copy), p(d), p(out), rows, C, 1, 1, cp, 1, st) == 0
+        assert torch.equal(out, w)
+    out.fill_(-1.0)
+    assert lib.cf_tokens_to_f32(p(copy), p(out), rows, C, cp, st) == 0
     assert torch.equal(out, want)
