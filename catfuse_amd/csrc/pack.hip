@@ -26,23 +26,27 @@ struct __attribute__((packed, aligned(4))) f32x4u {
   float v[4];
 };
 
-// Workgroup: 64 pixels x a run of 64-channel tiles.  Bound by HBM; what it
-// needs is bytes in flight, so a tile's sixteen floats a thread are loaded
-// together (four 16-byte loads along the pixels: two channel pairs of four
-// pixels), and without `act` (whose bits need a pixel's every channel in one
-// workgroup) each 64-channel tile is a workgroup of its own (grid z).  A
-// channel pair's halves are one LDS word, in rows of 33 words a pixel: the
-// transposing writes and the row reads both touch every bank alike.
+// Workgroup: 64 pixels x a run of TC-channel tiles (64, or 32 for copies of one
+// 32-channel group).  Bound by HBM; what it needs is bytes in flight, so a tile's
+// floats of a thread are loaded together (TC = 64: four 16-byte loads along the
+// pixels, two channel pairs of four pixels), and without `act` (whose bits need a
+// pixel's every channel in one workgroup) each tile is a workgroup of its own
+// (grid z).  A channel pair's halves are one LDS word, in rows of TC / 2 + 1 words a
+// pixel: the transposing writes and the row reads both touch every bank alike.
 // Measured (MI355X), against one workgroup walking a pixel block's channels
 // 32 at a time with 4-byte loads: 128 images of 256 x 14 x 14 33.4 -> 12.1 us,
 // of 64 x 56 x 56 (154 MB moved) 61 -> 29.6 us.
-template <bool ACT>
+template <bool ACT, int TC>
 __global__ __launch_bounds__(256) void pack_kernel(
     const float* __restrict__ x, int64_t C, int64_t HW, int64_t Cp, _Float16* __restrict__ xp,
     uint32_t* __restrict__ act, int gs, float thr, unsigned long long* __restrict__ nnz,
     uint32_t* __restrict__ status) {
   typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-  constexpr int TC = 64, LD = TC / 2 + 1;   // channels of a tile; words of a pixel's row
+  constexpr int LD = TC / 2 + 1;   // words of a pixel's row
+  constexpr int NI = TC / 32;      // channel pairs of a thread
+  // Channels past C neither loaded nor converted: of one group they may be most;
+  // in a run of tiles the branch costs more (2 x 2048 x 56 x 56 with `act` 58 -> 65 us).
+  constexpr bool SKIP = TC == 32;
   __shared__ uint32_t tile[PX * LD];
   __shared__ uint32_t bits_sh[PX];
   __shared__ unsigned int cnt_sh;
@@ -61,14 +65,17 @@ __global__ __launch_bounds__(256) void pack_kernel(
   const float* xn = x + n * C * HW + hw0 + p0;
   __syncthreads();
   for (int64_t c0 = (int64_t)blockIdx.z * TC; c0 < Cp; c0 += (int64_t)gridDim.z * TC) {
-    float v[2][2][4];
+    float v[NI][2][4];
 #pragma unroll
-    for (int i = 0; i < 2; ++i)
+    for (int i = 0; i < NI; ++i)
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
         const int64_t c = c0 + 2 * (cr + 16 * i) + u;
         const float* src = xn + c * HW;
-        if (c < C && left >= 4) {
+        if (SKIP && c >= C) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) v[i][u][j] = 0.0f;
+        } else if (c < C && left >= 4) {
           const f32x4u q = *reinterpret_cast<const f32x4u*>(src);
 #pragma unroll
           for (int j = 0; j < 4; ++j) v[i][u][j] = q.v[j];
@@ -78,8 +85,13 @@ __global__ __launch_bounds__(256) void pack_kernel(
         }
       }
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
+    for (int i = 0; i < NI; ++i) {
       const int w = cr + 16 * i;
+      if (SKIP && c0 + 2 * w >= C) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) tile[(p0 + j) * LD + w] = 0u;
+        continue;
+      }
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         h2 h;
@@ -100,10 +112,10 @@ __global__ __launch_bounds__(256) void pack_kernel(
     }
     __syncthreads();
     if (xp) {
-      // write phase: 8 threads per pixel, 8 channels (16 B) each
+      // write phase: TC / 8 threads per pixel, 8 channels (16 B) each
 #pragma unroll
-      for (int i = 0; i < 2; ++i) {
-        const int wp = tid / 8 + 32 * i, part = tid % 8;
+      for (int i = 0; i < NI; ++i) {
+        const int wp = tid / (TC / 8) + 32 * i, part = tid % (TC / 8);
         if (hw0 + wp < HW && c0 + part * 8 < Cp) {
           const uint32_t* r = &tile[wp * LD + part * 4];
           *reinterpret_cast<uint4*>(xp + ((n * HW + hw0 + wp) * Cp + c0 + part * 8)) =
@@ -681,12 +693,16 @@ CF_API int cf_pack_input(const float* x, int64_t NB, int64_t C, int64_t H, int64
   if (nnz && (unsigned long long)grid.x * grid.y * grid.z >= CF_MAX_COUNT_WG)
     grid.z = 1;   // one workgroup walks the channels
   if (nnz && (unsigned long long)grid.x * grid.y >= CF_MAX_COUNT_WG) return (int)hipErrorInvalidValue;
-  if (act)
-    hipLaunchKernelGGL(pack_kernel<true>, grid, dim3(256), 0, (hipStream_t)stream, x, C, HW,
-                       Cp, (_Float16*)xp, act, group_size, threshold, nnz, status);
-  else
-    hipLaunchKernelGGL(pack_kernel<false>, grid, dim3(256), 0, (hipStream_t)stream, x, C, HW,
-                       Cp, (_Float16*)xp, act, group_size, threshold, nnz, status);
+#define CF_PACK(ACT, TC)                                                                          \
+  hipLaunchKernelGGL((pack_kernel<ACT, TC>), grid, dim3(256), 0, (hipStream_t)stream, x, C, HW, Cp, \
+                     (_Float16*)xp, act, group_size, threshold, nnz, status)
+  // (copies of at most 32 channels, 64- / 32-channel tiles: 16 x 3 x 224 x 224 with
+  // activity bits 39 / 23.6 us, without 25 / 20.1)
+  if (act && Cp <= 32) CF_PACK(true, 32);
+  else if (act) CF_PACK(true, 64);
+  else if (Cp <= 32) CF_PACK(false, 32);
+  else CF_PACK(false, 64);
+#undef CF_PACK
   return (int)hipGetLastError();
 }
 
