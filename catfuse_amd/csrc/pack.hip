@@ -15,6 +15,8 @@
 // prescan.hip.  HBM traffic: 4 B read + 2 B (xp) + 4/C B (act) per element.
 #include "cf_common.h"
 
+#include <type_traits>
+
 namespace {
 
 constexpr int PX = 64;   // pixels per block
@@ -508,13 +510,48 @@ __global__ __launch_bounds__(256) void tokens_to_f32_chunks_kernel(
 // Linear-LIF): out[m][o] = bias[o] + sum_k x[m][k] * w[o][k] in fp32, x read
 // through the copy's output descriptor (an all-zero copy gives the bias).
 // One workgroup per row: its 256 threads take every 256th k (coalesced
-// weight rows), LT_OB outputs a pass; the partial sums are reduced in a
+// weight rows), OB outputs a pass; the partial sums are reduced in a
 // fixed tree (lanes, then waves in order), so the result is deterministic.
 // Spike values are small integers; a zero leaves the sums as they are (exact,
-// whatever the weight).  Bound by latency: a thread loads the weights of LT_KB
-// k's together, whether or not their spikes are zero (VGG-11's head, 256 rows
-// of 4096 -> 10: 48.6 -> 13 us, where each k waited for its own).
-constexpr int LT_OB = 16, LT_KB = 4;
+// whatever the weight).  Bound by latency: a thread loads the weights of KB
+// k's together, beside their spikes (VGG-11's head, 256 rows of 4096 -> 10: 48.6 ->
+// 13 us, where each k waited for its own).  At every output pass after the first
+// a wave skips the groups of KB k's whose spikes are all zero in it (`live`, a bit
+// a group): 32 silent rows of 2048 -> 1000 334 us without, 125 so.  (In the first
+// pass a silent row costs what a live one does: 256 rows of 2048 -> 10 6.4 us, where
+// looking at the spikes first takes silent ones 5.8 and live ones 7.0.)  OB 4 for a
+// last pass of few outputs, KB 1 or 2 for rows of at most 256 or 512: no loads of
+// weights that are not used (1024 rows of 2048 -> 1 11.0 -> 6.7 us).
+template <int OB, int KB>
+__device__ __forceinline__ void linear_tokens_sum(const _Float16* __restrict__ xr,
+                                                  const float* __restrict__ w, int K, int no,
+                                                  bool first, uint64_t& live, float* acc) {
+  int g = 0;
+  for (int k0 = threadIdx.x; k0 < K; k0 += 256 * KB, ++g) {
+    if (!first && g < 64 && ((live >> g) & 1ull) == 0ull) continue;
+    float xv[KB], wv[KB][OB];
+#pragma unroll
+    for (int u = 0; u < KB; ++u) {
+      const int k = k0 + 256 * u;
+      xv[u] = k < K ? (float)xr[k] : 0.0f;
+      // (a row or column beyond the matrix repeats one inside it, unused)
+      const float* wk = w + (k < K ? k : k0);
+#pragma unroll
+      for (int j = 0; j < OB; ++j) wv[u][j] = wk[(size_t)(j < no ? j : 0) * K];
+    }
+    bool nz = false;
+#pragma unroll
+    for (int u = 0; u < KB; ++u) {
+      nz |= xv[u] != 0.0f;
+#pragma unroll
+      for (int j = 0; j < OB; ++j) acc[j] = xv[u] != 0.0f ? fmaf(xv[u], wv[u][j], acc[j]) : acc[j];
+    }
+    if (first && g < 64 && __any(nz ? 1 : 0)) live |= 1ull << g;
+  }
+}
+
+constexpr int LT_OB = 16;
+template <int KB>
 __global__ __launch_bounds__(256) void linear_tokens_kernel(
     const _Float16* __restrict__ xp, const CfOutDesc* __restrict__ desc,
     const float* __restrict__ w, const float* __restrict__ bias, float* __restrict__ out,
@@ -523,44 +560,33 @@ __global__ __launch_bounds__(256) void linear_tokens_kernel(
   const int m = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const _Float16* xs = cf_copy_source(desc, xp);
   const _Float16* xr = xs != nullptr ? xs + (size_t)m * cp : nullptr;
-  for (int o0 = 0; o0 < O; o0 += LT_OB) {
-    float acc[LT_OB];
+  uint64_t live = 0ull;
+  auto pass = [&](auto ob_c, int o0) {
+    constexpr int OB = decltype(ob_c)::value;
+    const float* wo = w + (size_t)o0 * K;
+    const int no = O - o0 < OB ? O - o0 : OB;
+    float acc[OB];
 #pragma unroll
-    for (int j = 0; j < LT_OB; ++j) acc[j] = 0.0f;
-    if (xr != nullptr) {
-      const int no = O - o0 < LT_OB ? O - o0 : LT_OB;
-      for (int k0 = tid; k0 < K; k0 += 256 * LT_KB) {
-        float xv[LT_KB], wv[LT_KB][LT_OB];
+    for (int j = 0; j < OB; ++j) acc[j] = 0.0f;
+    if (xr != nullptr) linear_tokens_sum<OB, KB>(xr, wo, K, no, o0 == 0, live, acc);
 #pragma unroll
-        for (int u = 0; u < LT_KB; ++u) {
-          const int k = k0 + 256 * u;
-          xv[u] = k < K ? (float)xr[k] : 0.0f;
-          // (a row or column beyond the matrix repeats one inside it, unused)
-          const float* wk = w + (size_t)o0 * K + (k < K ? k : k0);
-#pragma unroll
-          for (int j = 0; j < LT_OB; ++j) wv[u][j] = wk[(size_t)(j < no ? j : 0) * K];
-        }
-#pragma unroll
-        for (int u = 0; u < LT_KB; ++u)
-#pragma unroll
-          for (int j = 0; j < LT_OB; ++j)
-            acc[j] = xv[u] != 0.0f ? fmaf(xv[u], wv[u][j], acc[j]) : acc[j];
-      }
-    }
-#pragma unroll
-    for (int j = 0; j < LT_OB; ++j)
+    for (int j = 0; j < OB; ++j)
 #pragma unroll
       for (int off = 32; off >= 1; off >>= 1) acc[j] += __shfl_xor(acc[j], off, 64);
     if (lane == 0) {
 #pragma unroll
-      for (int j = 0; j < LT_OB; ++j) red[wave][j] = acc[j];
+      for (int j = 0; j < OB; ++j) red[wave][j] = acc[j];
     }
     __syncthreads();
-    if (tid < LT_OB && o0 + tid < O) {
+    if (tid < OB && o0 + tid < O) {
       const float s = ((red[0][tid] + red[1][tid]) + red[2][tid]) + red[3][tid];
       out[(size_t)m * O + o0 + tid] = bias != nullptr ? bias[o0 + tid] + s : s;
     }
     __syncthreads();   // red is rewritten by the next pass
+  };
+  for (int o0 = 0; o0 < O; o0 += LT_OB) {
+    if (O - o0 > 4) pass(std::integral_constant<int, LT_OB>{}, o0);
+    else pass(std::integral_constant<int, 4>{}, o0);
   }
 }
 
@@ -920,9 +946,14 @@ CF_API int cf_linear_tokens(const void* xp, const void* desc, const float* w, co
       O > 4096 || K * O > INT32_MAX || (int64_t)M * cp > ((int64_t)1 << 40))
     return (int)hipErrorInvalidValue;
   if (M == 0) return 0;
-  hipLaunchKernelGGL(linear_tokens_kernel, dim3((unsigned)M), dim3(256), 0, (hipStream_t)stream,
-                     (const _Float16*)xp, (const CfOutDesc*)desc, w, bias, out, (int)K, (int)cp,
-                     (int)O);
+#define CF_LINEAR(KB)                                                                         \
+  hipLaunchKernelGGL(linear_tokens_kernel<KB>, dim3((unsigned)M), dim3(256), 0,               \
+                     (hipStream_t)stream, (const _Float16*)xp, (const CfOutDesc*)desc, w, bias, \
+                     out, (int)K, (int)cp, (int)O)
+  if (K <= 256) CF_LINEAR(1);
+  else if (K <= 512) CF_LINEAR(2);
+  else CF_LINEAR(4);
+#undef CF_LINEAR
   return (int)hipGetLastError();
 }
 

@@ -51,6 +51,29 @@ def _check_attention(cuda, N, T, B, heads, cp_pad):
         assert torch.equal(vo, v_out)
 
 
+@pytest.mark.parametrize("K,O", [(300, 21), (70000, 18)])
+def test_linear_tokens_silent_rows(cuda, K, O):
+    """Rows silent but for one spike (skipped groups of inputs at every output
+    pass but the first), a wholly silent one, a copy recorded as all zero."""
+    from catfuse_amd import runtime
+    g = torch.Generator().manual_seed(K)
+    at = [0, 63, 64, K // 2, K - 1]
+    x = torch.zeros(1, len(at) + 1, K)
+    x[0, range(len(at)), at] = 2.0
+    w, b = torch.randn(O, K, generator=g), torch.randn(O, generator=g)
+    copy = runtime.pack_tokens(x.to(cuda), runtime.pad32(K))
+    y = runtime.linear_tokens(runtime.lazy_tokens(x.shape, copy, torch.device(cuda)), w.to(cuda),
+                              b.to(cuda)).cpu()
+    # one product of two, exact, and one addition
+    assert torch.equal(y[0], torch.cat([b + 2.0 * w[:, at].t(), b[None]]))
+    p, lib = runtime.ptr, runtime._hip.lib()
+    zero = torch.tensor([1, 0], dtype=torch.int64, device=cuda)
+    out, wg, bg = torch.empty(len(at) + 1, O, device=cuda), w.to(cuda), b.to(cuda)
+    assert lib.cf_linear_tokens(p(copy), p(zero), p(wg), p(bg), p(out), len(at) + 1, K,
+                                runtime.pad32(K), O, runtime._hip.stream(out.device)) == 0
+    assert torch.equal(out.cpu(), b.expand(len(at) + 1, O))
+
+
 @pytest.mark.parametrize("K,O", [(1, 1), (255, 10), (1024, 16), (1025, 17), (4096, 40), (5000, 3)])
 def test_linear_tokens_edges(cuda, K, O):
     from catfuse_amd import runtime
