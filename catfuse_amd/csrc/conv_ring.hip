@@ -696,7 +696,8 @@ bool cf_conv_ring(int* rc, const void* x, const void* w_packed, const float* alp
     if (T <= 4 && H >= 4 && W >= 4) {
       const int64_t nch = Cp / KC;
       const int64_t halo_wg = B * ((H + 7) / 8) * ((W + 7) / 8) * (Coutp / 64);
-      if (nch + T < 5 || (n32 > cus && halo_wg <= cus && nch < 7)) return false;
+      if (nch + T < 5 || (n32 > cus && halo_wg <= cus && nch < (T < 4 ? 7 : 6)))
+        return false;
     }
     mw = n32 <= cus ? 1 : 2;
   }

@@ -411,20 +411,19 @@ __global__ __launch_bounds__(256) void pack_tokens_kernel(
 #pragma unroll
       for (int k = 0; k < U; ++k) {
         const int64_t u = u0 + k * step;
-        dst[k] = -1;
-        if (k > 0 && u >= units) continue;
+        const bool live = u < units;
         const int64_t r = small ? (int64_t)((uint32_t)u / nc8) : u / nc8;
         const int c0 = (int)(u - r * nc8) * 8;
-        dst[k] = r * cp + c0;
+        dst[k] = live ? r * cp + c0 : -1;
         const float* src = x + r * C + c0;
-        if (c0 + 8 <= C) {
+        if (live && c0 + 8 <= C) {
           const f32x4u q0 = *reinterpret_cast<const f32x4u*>(src);
           const f32x4u q1 = *reinterpret_cast<const f32x4u*>(src + 4);
 #pragma unroll
           for (int j = 0; j < 4; ++j) { v[k][j] = q0.v[j]; v[k][4 + j] = q1.v[j]; }
         } else {
 #pragma unroll
-          for (int j = 0; j < 8; ++j) v[k][j] = c0 + j < C ? src[j] : 0.0f;
+          for (int j = 0; j < 8; ++j) v[k][j] = (live && c0 + j < C) ? src[j] : 0.0f;
         }
       }
 #pragma unroll
@@ -791,17 +790,18 @@ static int nhwc_to_nchw(const void* xp, const void* desc, float* out, int64_t NB
   const int64_t HW = H * W;
   // The wide form where its tiles waste no half (an even number of 32-channel
   // groups) and either maps are so small that a tile is mostly channels, or an
-  // fp16 copy is so large that HBM is what bounds it; rows of about 4 KB and its
-  // multiples put its 16 channels' stores on the same channels of the memory.
-  // Measured (us, 32 channels / wide): 488 x 512 channels of 2 x 2 8.3 / 6.4, 3906 x
-  // 256 of 1 x 1 25 / 14.4; 298 x 512 of 14 x 14 47.5 / 40, 149 x 64 of 56 x 56 35.5 /
-  // 30.3, but 59 x 512 of 14 x 14 11 / 11, 71 x 90 of 32 x 32 7.7 / 11.2, 742 x 40 of
-  // 30 x 34 37.2 / 39.8, 128 x 512 of 7 x 7 5.5 / 6.5, 49 x 332 of 10 x 10 4.5 / 5.2,
-  // bytes of 128 x 256 of 14 x 14 9.9 / 11.3.
+  // fp16 copy is so large that the traffic is what bounds it; rows of about 4 KB and
+  // its multiples put its 16 channels' stores on the same channels of the memory.
+  // Measured after another pass has used the L2 (us, 32 channels / wide): 128 x 256
+  // channels of 14 x 14 11.2 / 10.9, 128 x 128 of 28 x 28 16.6 / 14.7, 364 x 48 of 33 x 32
+  // 26.0 / 21.7, but 32 x 384 of 14 x 14 5.5 / 6.2, 32 x 64 of 32 x 32 4.1 / 4.6, 128 x 512
+  // of 7 x 7 6.0 / 6.7, 4096 x 64 of 6 x 5 11.2 / 13.4; one pass after another: 488 x 512
+  // of 2 x 2 8.3 / 6.4, 3906 x 256 of 1 x 1 25 / 14.4, 742 x 40 of 30 x 34 37.2 / 39.8, bytes
+  // of 128 x 256 of 14 x 14 9.9 / 11.3.
   const int64_t tiles = (HW + PX - 1) / PX * ((C + 63) / 64) * NB;
   const bool wide = (C + CC - 1) / CC % 2 == 0 &&
                     (HW <= 16 ? tiles >= 900
-                              : sizeof(XT) == 2 && HW >= 100 && (HW + 32) % 1024 > 64 && tiles >= 3000);
+                              : sizeof(XT) == 2 && HW >= 100 && (HW + 16) % 1024 > 32 && tiles >= 1700);
   if (wide)
     hipLaunchKernelGGL(nhwc_to_nchw_wide_kernel<XT>,
                        dim3(cf_blocks(HW, PX), (unsigned)((C + 63) / 64), (unsigned)NB), dim3(256),
@@ -820,11 +820,12 @@ static int tokens_to_f32(const void* xp, const void* desc, float* out, int64_t r
   if (!xp || !out || rows < 0 || C <= 0 || cp < C || rows * cp > ((int64_t)1 << 40))
     return (int)hipErrorInvalidValue;
   if (rows == 0) return 0;
-  // Chunks where HBM bounds the pass: 50,176 rows of 384 26 -> 22 us; 3,136 of 384
-  // equal; rows that chunks do not fill cost a second, element-wise round: 784 rows
-  // of 100 2.6 -> 3.1, 100,000 of 33 6.5 -> 7.2, 50,176 of 257 19.3 -> 17.4.
+  // Chunks for rows that they fill (after another pass: 4 rows of 512 2.2 -> 1.8 us,
+  // 254 of 384 2.4 -> 2.2, 28,661 of 32 3.6 -> 3.0, 50,176 of 384 26 -> 22), but for rows of
+  // one (a million of 8 16.2 -> 18.5).  Others cost a second, element-wise round: 784
+  // rows of 100 2.6 -> 3.1, 100,000 of 33 6.5 -> 7.2; 50,176 of 257 19.3 -> 17.4.
   const int64_t n = rows * C;
-  const bool chunks = C % 8 == 0 ? n >= (1 << 21) : C >= 256 && n >= (1 << 23);
+  const bool chunks = C % 8 == 0 ? C >= 16 : C >= 256 && n >= (1 << 23);
   const int64_t units = chunks ? rows * ((C + 7) / 8) : n;
   const int64_t wg = (units + 255) / 256, most = chunks ? 16384 : 4096;
   const dim3 grid((unsigned)(wg < most ? wg : most));
@@ -916,12 +917,13 @@ CF_API int cf_pack_tokens(const float* x, int64_t rows, int64_t C, int64_t cp, v
     return (int)hipErrorInvalidValue;
   if (rows == 0) return 0;
   const int64_t units = rows * (cp / 8);
-  // Two chunks a thread once a launch has enough of them for its loads to bound it:
-  // 3,136 rows of 256 (100,352 chunks) 5.4 -> 4.4 us, 784 of 384 (37,632) equal; later
-  // where chunks are padding or partial: 12,544 rows of 48 (100,352) 4.4 -> 4.9, of 100
-  // (200,704) 6.5 -> 5.3.  (4,096 workgroups hold the card's loads in flight; more
-  // only add count-block atomics.)
-  if (C >= 32 && units >= (8 * C >= 7 * cp ? 65536 : 196608))
+  // Two chunks a thread for rows of whole channel groups (after another pass: 4 rows
+  // of 512 3.6 -> 3.1 us, 205 of 1536 4.5 -> 4.2, 94,149 of 64 15.3 -> 8.7).  Others have
+  // chunks of padding and partial ones, and gain by it only once loads bound the
+  // launch: 12,544 rows of 48 (100,352 chunks) 4.4 -> 4.9, of 100 (200,704) 6.5 -> 5.3.
+  // (4,096 workgroups hold the card's loads in flight; more only add count-block
+  // atomics.)
+  if (C % 32 == 0 || (C > 32 && units >= (8 * C >= 7 * cp ? 65536 : 196608)))
     hipLaunchKernelGGL(pack_tokens_kernel<2>,
                        dim3((unsigned)((units + 511) / 512 < 4096 ? (units + 511) / 512 : 4096)),
                        dim3(256), 0, (hipStream_t)stream, x, rows, (int)C, (int)cp, (_Float16*)xp,

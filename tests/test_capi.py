@@ -328,7 +328,7 @@ def test_flat_tile_kernel_bounds():
     for Ci in range(32, 320, 32):
         for T in (1, 4, 5):
             assert (conv_choice(T, 8, Ci, 512, 14, 14, 1)
-                    == (RING if T > 4 or Ci >= 224 else HALO_LEAN)), (Ci, T)
+                    == (RING if T > 4 or Ci >= (224 if T < 4 else 192) else HALO_LEAN)), (Ci, T)
             assert (conv_choice(T, 30, Ci, 704, 7, 7, 1)
                     == (RING if Ci // 32 + T >= 5 else HALO_LEAN)), (Ci, T)
     assert conv_choice(4, 512, 512, 4096, 1, 1, 1) == GENERAL            # several rounds, 1x1 map
