@@ -790,18 +790,19 @@ static int nhwc_to_nchw(const void* xp, const void* desc, float* out, int64_t NB
   const int64_t HW = H * W;
   // The wide form where its tiles waste no half (an even number of 32-channel
   // groups) and either maps are so small that a tile is mostly channels, or an
-  // fp16 copy is so large that the traffic is what bounds it; rows of about 4 KB and
-  // its multiples put its 16 channels' stores on the same channels of the memory.
-  // Measured after another pass has used the L2 (us, 32 channels / wide): 128 x 256
-  // channels of 14 x 14 11.2 / 10.9, 128 x 128 of 28 x 28 16.6 / 14.7, 364 x 48 of 33 x 32
-  // 26.0 / 21.7, but 32 x 384 of 14 x 14 5.5 / 6.2, 32 x 64 of 32 x 32 4.1 / 4.6, 128 x 512
-  // of 7 x 7 6.0 / 6.7, 4096 x 64 of 6 x 5 11.2 / 13.4; one pass after another: 488 x 512
-  // of 2 x 2 8.3 / 6.4, 3906 x 256 of 1 x 1 25 / 14.4, 742 x 40 of 30 x 34 37.2 / 39.8, bytes
-  // of 128 x 256 of 14 x 14 9.9 / 11.3.
+  // fp16 copy is so large that the traffic is what bounds it.  Rows of a multiple
+  // of 2 KB, or up to 256 bytes less, put the stores of its 16 channels on the same
+  // channels of the memory.  Measured after another pass has used the L2 (us, 32
+  // channels / wide): 128 x 256 channels of 14 x 14 11.2 / 10.9, 128 x 128 of 28 x 28
+  // 16.6 / 14.7, 364 x 48 of 33 x 32 26.0 / 21.7, 30 x 170 of 23 x 31 7.6 / 7.4; but 32 x 384
+  // of 14 x 14 5.5 / 6.2, 189 x 64 of 19 x 24 7.3 / 8.9, 32 x 64 of 32 x 32 4.1 / 4.6, 128 x
+  // 512 of 7 x 7 6.0 / 6.7, 4096 x 64 of 6 x 5 11.2 / 13.4; one pass after another: 488 x
+  // 512 of 2 x 2 8.3 / 6.4, 3906 x 256 of 1 x 1 25 / 14.4, bytes of 128 x 256 of 14 x 14
+  // 9.9 / 11.3.
   const int64_t tiles = (HW + PX - 1) / PX * ((C + 63) / 64) * NB;
   const bool wide = (C + CC - 1) / CC % 2 == 0 &&
                     (HW <= 16 ? tiles >= 900
-                              : sizeof(XT) == 2 && HW >= 100 && (HW + 16) % 1024 > 32 && tiles >= 1700);
+                              : sizeof(XT) == 2 && HW >= 100 && (HW - 1) % 512 < 447 && tiles >= 1050);
   if (wide)
     hipLaunchKernelGGL(nhwc_to_nchw_wide_kernel<XT>,
                        dim3(cf_blocks(HW, PX), (unsigned)((C + 63) / 64), (unsigned)NB), dim3(256),
