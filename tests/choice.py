@@ -31,8 +31,7 @@ def conv_args(T, B, Ci, Co, H, W, k, stride=1, pool=False, ident=False, state=Tr
 
 def conv_choice(*args, **kw):
     """The kernel's number, or None for a launch that is refused."""
-    c = ctypes.c_int(-1)
-    rc = _hip.lib().cf_conv_mfma_choice(ctypes.addressof(conv_args(*args, **kw)),
-                                        ctypes.addressof(c))
+    a, c = conv_args(*args, **kw), ctypes.c_int(-1)     # (held until the call returns)
+    rc = _hip.lib().cf_conv_mfma_choice(ctypes.addressof(a), ctypes.addressof(c))
     assert rc in (0, 1)            # hipErrorInvalidValue
     return None if rc else c.value

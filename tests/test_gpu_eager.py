@@ -206,3 +206,49 @@ def test_repeat_path_matches_general_path_spikformer(cuda, monkeypatch, v_th):
         assert len(sf) == len(sg)
         for k, (a, b) in enumerate(zip(sf, sg)):
             assert torch.equal(a, b), f"input {i}: state of layer {k}"
+
+
+@pytest.mark.parametrize("pool", [False, True])
+def test_plain_inputs_match_general_path(cuda, monkeypatch, pool):
+    """A layer on plain fp32 inputs of two shapes in turn (one packing workspace,
+    a plan a shape), live and all zero, contiguous and not: outputs read after the
+    last call and states equal the general path's bit for bit, the plan taken by
+    every contiguous input."""
+    from catfuse_amd import runtime
+    g = torch.Generator().manual_seed(5)
+    w = (torch.randn(64, 40, 3, 3, generator=g) * 0.1).to(cuda)
+    sh = (torch.randn(64, generator=g) * 0.1).to(cuda)
+    r = runtime.ConvLIFRunner(w, None, None, sh, 1, 1, 2.0, 0.4, 0.0, True)
+    a, a2 = ((torch.rand(4, 2, 40, 8, 8, generator=g) < 0.3).float().to(cuda) for _ in range(2))
+    b = (torch.rand(6, 1, 40, 10, 12, generator=g) < 0.3).float().to(cuda)
+    xs = [a, b, a2, torch.zeros_like(a), b.transpose(3, 4).contiguous().transpose(3, 4), a, b]
+    taken = []
+    repeat = runtime.ConvLIFRunner._dense_repeat
+
+    def count(self, *args, **kw):
+        res = repeat(self, *args, **kw)
+        taken.append(res is not None)
+        return res
+
+    monkeypatch.setattr(runtime.ConvLIFRunner, "_dense_repeat", count)
+    epi = runtime.EPI_POOL if pool else runtime.EPI_LIF
+
+    def run():
+        res = []
+        for x in xs:
+            if x.is_contiguous():
+                res.append(r.run_mfma(x, epilogue=epi))
+            else:
+                with pytest.raises(RuntimeError, match="contiguous"):
+                    r.run_mfma(x, epilogue=epi)
+        return [(y.clone(), v.clone()) for y, v in res]
+    fast = run()
+    assert taken == [x.is_contiguous() for x in xs]
+    runtime.REPEAT_PLANS = False
+    try:
+        general = run()
+    finally:
+        runtime.REPEAT_PLANS = True
+    for (ya, va), (yb, vb) in zip(fast, general):
+        assert torch.equal(ya, yb) and torch.equal(va, vb)
+    assert not torch.equal(fast[0][0], fast[2][0]) and bool(fast[0][0].any())

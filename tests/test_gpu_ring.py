@@ -32,12 +32,18 @@ POOLED = [(4, 1, 64, 64, 16, 16), (4, 3, 96, 64, 8, 8), (6, 5, 64, 64, 4, 4),
           (4, 33, 64, 96, 2, 2), (3, 2, 32, 32, 6, 4), (1, 4, 512, 512, 2, 2)]
 
 
-def _layer(cuda, Ci, Co, k, seed=0):
+# tau, v_th, v_reset, decay_input: the specialised hard reset off 0 and the generic
+# neuron (tau not a power of two, soft reset, no input decay); NEURONS[-1] fires at rest
+NEURONS = [(2.0, 0.3, 0.1, True), (3.0, 0.3, 0.0, True), (2.0, 0.3, None, True),
+           (2.0, 0.3, 0.0, False), (2.0, 0.05, 0.1, True)]
+
+
+def _layer(cuda, Ci, Co, k, seed=0, neuron=(2.0, 0.3, 0.0, True)):
     g = torch.Generator().manual_seed(seed)
     w = torch.randn(Co, Ci, k, k, generator=g) * (2.0 / (Co * k * k)) ** 0.5
     sc = torch.rand(Co, generator=g) * 0.4 + 0.8
     sh = torch.randn(Co, generator=g) * 0.1
-    r = ConvLIFRunner(w.to(cuda), sc.to(cuda), sh.to(cuda), None, 1, k // 2, 2.0, 0.3, 0.0, True)
+    r = ConvLIFRunner(w.to(cuda), sc.to(cuda), sh.to(cuda), None, 1, k // 2, *neuron)
     return r, w, sc, sh
 
 
@@ -108,6 +114,53 @@ def test_flat_tiles_pooled(cuda, shape, vin):
     ty, tv = _tiled(r, xl, v0, True, None)
     assert torch.equal(y.clone(), ty) and torch.equal(v.clone(), tv)
     assert 0 < float(y.mean()) < 1
+
+
+@pytest.mark.parametrize("neuron", NEURONS)
+@pytest.mark.parametrize("T,k,H,W,pool", [(6, 1, 5, 7, False), (5, 3, 9, 11, False), (4, 3, 8, 4, True)])
+def test_flat_tiles_neurons(cuda, neuron, T, k, H, W, pool):
+    """Every LIF specialisation of the flat-tile kernel, from a state, against the
+    8x8-tile kernel bit for bit and the neuron as it is defined."""
+    B, Ci, Co = 3, 64, 64
+    r, w, sc, sh = _layer(cuda, Ci, Co, k, neuron=neuron)
+    assert conv_choice(T, B, Ci, Co, H, W, k, pool=pool, lif=r.lif) == RING
+    g = torch.Generator().manual_seed(4)
+    x = (torch.rand(T, B, Ci, H, W, generator=g) < 0.3).float()
+    xl = _lazy(x, cuda)
+    Hs, Ws = (H // 2, W // 2) if pool else (H, W)
+    v0 = torch.rand(B, Co, Hs, Ws, generator=g) * 0.25
+    y, v = r.run_mfma(xl, v0.to(cuda), epilogue=EPI_POOL if pool else EPI_LIF)
+    ty, tv = _tiled(r, xl, v0.to(cuda), pool, None)
+    assert torch.equal(y.clone(), ty) and torch.equal(v.clone(), tv)
+    z = torch.as_tensor(np.asarray(oracle.conv2d(x.reshape(T * B, Ci, H, W), w, None, 1, k // 2)))
+    z = (z.reshape(T * B, Co, H, W) * sc.view(-1, 1, 1) + sh.view(-1, 1, 1)).float()
+    if pool:
+        z = torch.nn.functional.avg_pool2d(z, 2)
+    tau, v_th, v_reset, decay = neuron
+    s_ref, v_ref, h_ref = oracle.lif_multistep(z.reshape(T, B, Co, Hs, Ws), v0, tau=tau,
+                                               v_threshold=v_th, v_reset=v_reset,
+                                               decay_input=decay)
+    lif_parity(ty.cpu().numpy(), tv.cpu().numpy(), s_ref, v_ref, h_ref, v_th=v_th)
+
+
+@pytest.mark.parametrize("neuron", NEURONS)
+@pytest.mark.parametrize("Co", [5, 70])
+def test_channels_off_32_neurons(cuda, neuron, Co):
+    """The 8x8-tile kernel off 32 channels with other neurons: those silent at rest
+    take the lean epilogue and leave the copy's padding zero, whatever they reset
+    to; all give the bits of the general epilogue with fp32 output."""
+    T, B, Ci, H, W = 5, 2, 48, 19, 65
+    r = _layer(cuda, Ci, Co, 3, neuron=neuron)[0]
+    silent = neuron is not NEURONS[-1]
+    assert conv_choice(T, B, Ci, Co, H, W, 3, lif=r.lif) == (HALO_LEAN if silent else HALO)
+    g = torch.Generator().manual_seed(Co)
+    xl = _lazy((torch.rand(T, B, Ci, H, W, generator=g) < 0.3).float(), cuda)
+    v0 = (torch.rand(B, Co, H, W, generator=g) * 0.25).to(cuda)
+    for v_in in (None, v0):
+        y, v = r.run_mfma(xl, v_in)
+        assert bool(y._cf_nhwc[0][..., Co:].any()) != silent
+        gy, gv = r.run_mfma(xl, v_in, emit_nhwc=False)
+        assert torch.equal(y.clone(), gy) and torch.equal(v.clone(), gv)
 
 
 @pytest.mark.parametrize("k,pool", [(1, False), (3, False), (3, True)])
