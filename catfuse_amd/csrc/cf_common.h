@@ -197,8 +197,10 @@ __device__ __forceinline__ void cf_count_publish(unsigned long long* blk, unsign
   }
 }
 
-// Workgroup "any" of a per-thread predicate (256-thread workgroups): one
-// wave vote per wave, combined through four LDS words after a barrier.
+// Workgroup "any" of a per-thread predicate: one wave vote per wave, the first
+// four waves' combined through LDS words after a barrier.  A wave beyond the
+// fourth (the weight-copying one of conv_ring.hip) only joins the barrier, with
+// false and a word of its own in sh4.
 __device__ __forceinline__ bool cf_wg_any(bool pred, unsigned* sh4) {
   const bool w = __any(pred ? 1 : 0) != 0;
   if ((threadIdx.x & 63) == 0) sh4[threadIdx.x >> 6] = w ? 1u : 0u;

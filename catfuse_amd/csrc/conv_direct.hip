@@ -165,9 +165,15 @@ struct DirectPoolArgs {
   LifParams lif;
 };
 
-template <int COB, int LM, bool FAST>
+// Output channels a workgroup.  Sixteen are 91 VGPRs with FAST, 103 to 105 without:
+// five and four waves a SIMD to hide the scalar loads and the barriers behind; a
+// wider group would hold z and v of more channels at two.
+constexpr int DP_COB = 16;
+
+template <int LM, bool FAST>
 __global__ __launch_bounds__(256) void conv_direct_pool_kernel(DirectPoolArgs a) {
-  static_assert(COB % 8 == 0 && COB <= 64, "8 channels a word");
+  constexpr int COB = DP_COB;
+  static_assert(COB % 8 == 0, "8 channels a word");
   static_assert(!FAST || LM == LM_HARD0_DECAY_P2, "reset-free charges: a hard reset to +0");
   constexpr int NWD = COB / 8;
   __shared__ float xs[DP_MAXCIN][DP_XH][DP_XW];
@@ -521,7 +527,7 @@ hipError_t launch_direct_pool(const DirectPoolArgs& a, dim3 grid, hipStream_t st
   const bool fast = lm == LM_HARD0_DECAY_P2 && a.T == 4 && a.x_img_tstride == 0 && !a.v_in &&
                     a.lif.inv_tau > 0.0f && a.lif.inv_tau <= 1.0f;
 #define CF_DIRECT_POOL(LMV, F) \
-  hipLaunchKernelGGL((conv_direct_pool_kernel<16, LMV, F>), grid, dim3(256), 0, st, a)
+  hipLaunchKernelGGL((conv_direct_pool_kernel<LMV, F>), grid, dim3(256), 0, st, a)
   if (fast) CF_DIRECT_POOL(LM_HARD0_DECAY_P2, true);
   else if (lm == LM_HARD0_DECAY_P2) CF_DIRECT_POOL(LM_HARD0_DECAY_P2, false);
   else if (lm == LM_HARD_DECAY_P2) CF_DIRECT_POOL(LM_HARD_DECAY_P2, false);
@@ -588,12 +594,8 @@ CF_API int cf_conv_direct_lif_maxpool(const float* x, const float* wt, const flo
   if (Ho <= 0 || Wo <= 0) return (int)hipErrorInvalidValue;
   const int64_t Hp = (Ho - 1) / 2 + 1, Wp = (Wo - 1) / 2 + 1;
   const int64_t tiles_h = (Hp + DP_PH - 1) / DP_PH, tiles_w = (Wp + DP_PW - 1) / DP_PW;
-  // 16 channels a workgroup: 87 VGPRs, five waves a SIMD to hide the
-  // per-step barriers (wider groups hold z and v for more channels and run
-  // two waves a SIMD)
-  const int cob = Cout % 16 == 0 ? 16 : 0;
-  if (cob == 0 || tiles_h * tiles_w > 0x7fffffff) return (int)hipErrorInvalidValue;
-  const int64_t nwg = tiles_h * tiles_w * B * (Cout / cob);
+  if (Cout % DP_COB != 0 || tiles_h * tiles_w > 0x7fffffff) return (int)hipErrorInvalidValue;
+  const int64_t nwg = tiles_h * tiles_w * B * (Cout / DP_COB);
   if (nz_out && nwg >= (int64_t)CF_MAX_COUNT_WG) return (int)hipErrorInvalidValue;
   DirectPoolArgs a;
   a.x = x; a.wt = wt; a.alpha = alpha; a.beta = beta; a.v_in = v_in; a.v_out = v_out;
@@ -602,7 +604,7 @@ CF_API int cf_conv_direct_lif_maxpool(const float* x, const float* wt, const flo
   a.Ho = (int)Ho; a.Wo = (int)Wo; a.pad = (int)pad; a.Hp = (int)Hp; a.Wp = (int)Wp;
   a.tiles_w = (int)tiles_w; a.x_img_tstride = (int)x_img_tstride;
   a.lif = cf_make_lif_params(tau, v_th, v_reset, hard_reset, decay_input);
-  const dim3 grid((unsigned)(tiles_h * tiles_w), (unsigned)B, (unsigned)(Cout / cob));
+  const dim3 grid((unsigned)(tiles_h * tiles_w), (unsigned)B, (unsigned)(Cout / DP_COB));
   return (int)launch_direct_pool(a, grid, (hipStream_t)stream);
 }
 

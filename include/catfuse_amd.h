@@ -388,8 +388,9 @@ int cf_conv_mfma(const void* x, const void* w_packed, const float* alpha, const 
  * (tile_h x tile_w) output tile staged in LDS once per 32-channel chunk and
  * up to 4 time steps accumulated per tile (weights fetched once per tap for
  * all of them).  cf_conv_mfma forwards every 3x3 layer and every 1x1 layer
- * with Ho, Wo >= 4 here (tile 8x8 when tile_h = 0), so all routes and
- * epilogues of a layer accumulate in the same order.  ksize: 1 or 3.
+ * with Ho, Wo >= 4 here (tile 8x8 when tile_h = 0), but for the launches its
+ * flat-tile kernel is faster at (cf_conv_mfma_choice), which accumulates in
+ * the same order: all routes and epilogues of a layer do.  ksize: 1 or 3.
  * Tiles: 8x8, or 8x16 with stride 1 and ksize 3.  Other arguments as
  * cf_conv_mfma.  Replaces the same reference interfaces as cf_conv_mfma. */
 int cf_conv_halo(const void* x, const void* w_packed, const float* alpha, const float* beta,
