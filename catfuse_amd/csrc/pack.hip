@@ -516,18 +516,19 @@ __global__ __launch_bounds__(256) void tokens_to_f32_chunks_kernel(
 // k's together, beside their spikes (VGG-11's head, 256 rows of 4096 -> 10: 48.6 ->
 // 13 us, where each k waited for its own).  At every output pass after the first
 // a wave skips the groups of KB k's whose spikes are all zero in it (`live`, a bit
-// a group): 32 silent rows of 2048 -> 1000 334 us without, 125 so.  (In the first
-// pass a silent row costs what a live one does: 256 rows of 2048 -> 10 6.4 us, where
+// a group): 32 silent rows of 2048 -> 1000 334 us without, 124 so.  (In the first
+// pass a silent row costs what a live one does: 256 rows of 2048 -> 10 6.1 us, where
 // looking at the spikes first takes silent ones 5.8 and live ones 7.0.)  OB 4 for a
 // last pass of few outputs, KB 1 or 2 for rows of at most 256 or 512: no loads of
 // weights that are not used (1024 rows of 2048 -> 1 11.0 -> 6.7 us).
 template <int OB, int KB>
 __device__ __forceinline__ void linear_tokens_sum(const _Float16* __restrict__ xr,
                                                   const float* __restrict__ w, int K, int no,
-                                                  bool first, uint64_t& live, float* acc) {
+                                                  bool mark, bool skip, uint64_t& live,
+                                                  float* acc) {
   int g = 0;
   for (int k0 = threadIdx.x; k0 < K; k0 += 256 * KB, ++g) {
-    if (!first && g < 64 && ((live >> g) & 1ull) == 0ull) continue;
+    if (skip && g < 64 && ((live >> g) & 1ull) == 0ull) continue;
     float xv[KB], wv[KB][OB];
 #pragma unroll
     for (int u = 0; u < KB; ++u) {
@@ -545,7 +546,7 @@ __device__ __forceinline__ void linear_tokens_sum(const _Float16* __restrict__ x
 #pragma unroll
       for (int j = 0; j < OB; ++j) acc[j] = xv[u] != 0.0f ? fmaf(xv[u], wv[u][j], acc[j]) : acc[j];
     }
-    if (first && g < 64 && __any(nz ? 1 : 0)) live |= 1ull << g;
+    if (mark && g < 64 && __any(nz ? 1 : 0)) live |= 1ull << g;
   }
 }
 
@@ -567,7 +568,9 @@ __global__ __launch_bounds__(256) void linear_tokens_kernel(
     float acc[OB];
 #pragma unroll
     for (int j = 0; j < OB; ++j) acc[j] = 0.0f;
-    if (xr != nullptr) linear_tokens_sum<OB, KB>(xr, wo, K, no, o0 == 0, live, acc);
+    // (the first pass marks the live groups for those that follow)
+    if (xr != nullptr)
+      linear_tokens_sum<OB, KB>(xr, wo, K, no, o0 == 0 && O > LT_OB, o0 > 0, live, acc);
 #pragma unroll
     for (int j = 0; j < OB; ++j)
 #pragma unroll
